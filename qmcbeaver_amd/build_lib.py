@@ -11,16 +11,21 @@ CSRC = os.path.join(HERE, "csrc")
 OBJ = os.path.join(HERE, "_obj")
 LIB = os.path.join(HERE, "libqmcb_amd.so")
 SOURCES = ["basis.hip", "orbital_gemm.hip", "slater.hip", "jastrow.hip", "cusp.hip", "multidet.hip",
-           "walk_ae.hip", "qmcb_abi.cpp", "qmcb_stats.cpp", "qmcb_cusp.cpp"]
+           "walk_ae.hip", "walk.hip", "qmcb_abi.cpp", "qmcb_stats.cpp", "qmcb_cusp.cpp"]
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 FLAGS = ["--offload-arch=gfx950", "-O3", "-std=c++17", "-fPIC",
          "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
          "-Wno-pass-failed"]
+# walk.hip is one long loop body whose exp, log and address constants the
+# compiler would hoist out of the loop into registers it then spills (124
+# spilled at 256 VGPRs in the 128-column tile, none with these two)
+EXTRA = {"walk.hip": ["-mllvm", "-disable-machine-licm",
+                      "-mllvm", "-sink-insts-to-avoid-spills"]}
 
 
 def _compile(src: str, obj_dir: str = OBJ, extra=()) -> str:
     obj = os.path.join(obj_dir, os.path.splitext(src)[0] + ".o")
-    cmd = [HIPCC, *FLAGS, *extra, "-c", os.path.join(CSRC, src), "-o", obj]
+    cmd = [HIPCC, *FLAGS, *EXTRA.get(src, ()), *extra, "-c", os.path.join(CSRC, src), "-o", obj]
     r = subprocess.run(cmd, capture_output=True, text=True)
     if r.returncode != 0:
         raise RuntimeError(f"hipcc failed for {src}:\n{r.stderr}")

@@ -83,6 +83,12 @@ struct qmcb_ctx {
   std::map<std::pair<int, int>, std::pair<int, int>> gemm_tile;
   std::pair<int, int> gemm_force{0, 0};
   bool separate_propose = false;  // QMCB_SEPARATE_PROPOSE set at creation
+  // single-electron walk in one launch per run of steps (walk.hip)
+  bool walk = false;
+  int pade_mn = 0, pade_md = 0;   // most terms of any Pade function
+  bool pade_one = true;           // every one has one term in each polynomial
+  int np_shell = 0;               // primitives, each shell's counted once
+  float *Cw[2] = {nullptr, nullptr};  // FP32 coefficients as [kpad / 4][npad][4]
   size_t ts = 8, tx = 8, to = 8;  // bytes: derivative storage, GEMM operand, GEMM output
 
   // resident walker state
@@ -596,6 +602,13 @@ struct Engine {
     return QMCB_OK;
   }
 
+  // a run of single-electron steps in one launch
+  static qmcb_status walk(qmcb_ctx *ctx, const WalkArgs &a, const int *d_map, int num) {
+    if constexpr (sizeof(TX) >= 4)
+      TIMED("sm_move", (launch_walk<TS, TX>(a, d_map, num, ctx->stream)));
+    return QMCB_OK;
+  }
+
   static qmcb_status commit(qmcb_ctx *ctx, const MoveArgs &a, const int *d_map,
                             const uint8_t *d_mask, int num) {
     TIMED("commit", (launch_commit<TS, TO>(a, d_map, d_mask, num, ctx->stream)));
@@ -719,6 +732,9 @@ hipError_t upload(qmcb_ctx *ctx, const T **dst, const T *src, size_t count) {
   return e;
 }
 
+// padded function count of the walk's rows: FP32 ones run in three stages of 16
+int walk_kpad(int kpad, size_t tx) { return tx == 4 ? (kpad + 47) / 48 * 48 : kpad; }
+
 size_t plan_device_bytes(const qmcb_system *s, const qmcb_options *o);
 
 qmcb_status create_impl(const qmcb_system *s, const qmcb_options *o, qmcb_ctx *ctx) {
@@ -787,6 +803,7 @@ qmcb_status create_impl(const qmcb_system *s, const qmcb_options *o, qmcb_ctx *c
   d.nprim = ctx->nprim;
   Shells sh = make_shells(s);
   ctx->nshell = d.nshell = (int)sh.atom.size();
+  for (int np : sh.nprim) ctx->np_shell += np;
   QCHK(upload(ctx, &d.nuc_xyz, s->nuc_xyz, 3 * (size_t)ctx->nn));
   QCHK(upload(ctx, &d.nuc_z, s->nuc_z, (size_t)ctx->nn));
   QCHK(upload(ctx, &d.sh_atom, sh.atom.data(), sh.atom.size()));
@@ -823,6 +840,16 @@ qmcb_status create_impl(const qmcb_system *s, const qmcb_options *o, qmcb_ctx *c
   QCHK(upload(ctx, &d.en[0], s->en_up, (size_t)ctx->nn));
   QCHK(upload(ctx, &d.en[1], s->en_dn, (size_t)ctx->nn));
   QCHK(upload(ctx, &ctx->d_ee, d.ee, 3));  // for kernels that take no DevSystem
+  auto pade_terms = [&](const qmcb_pade &f) {
+    ctx->pade_mn = std::max(ctx->pade_mn, (int)f.n_num);
+    ctx->pade_md = std::max(ctx->pade_md, (int)f.n_den);
+    if (f.n_num != 1 || f.n_den != 1) ctx->pade_one = false;
+  };
+  for (int i = 0; i < 3; i++) pade_terms(d.ee[i]);
+  for (int i = 0; i < ctx->nn; i++) {
+    pade_terms(s->en_up[i]);
+    pade_terms(s->en_dn[i]);
+  }
   double vnn = 0.0;
   for (int i = 0; i < ctx->nn; i++)
     for (int j = i + 1; j < ctx->nn; j++) {
@@ -869,6 +896,10 @@ qmcb_status create_impl(const qmcb_system *s, const qmcb_options *o, qmcb_ctx *c
     QCHK(upload(ctx, (const double **)&ctx->d_ci, s->ci_coef, (size_t)ctx->ndet));
   }
 
+  ctx->walk = !ctx->multi && o->precision != QMCB_MIXED_BF16 &&
+              walk_fits(ctx->n[0], ctx->B, walk_kpad(ctx->kpad, ctx->tx), ctx->nn, ctx->nshell, ctx->np_shell,
+                        ctx->pade_mn, ctx->pade_md, ctx->tx);
+
   // ---- transposed, padded MO coefficients (active orbitals) in the operand type
   for (int sp = 0; sp < 2; sp++) {
     const int n = ctx->nact[sp];
@@ -895,6 +926,16 @@ qmcb_status create_impl(const qmcb_system *s, const qmcb_options *o, qmcb_ctx *c
       std::vector<float> cf(cnt);
       for (size_t i = 0; i < cnt; i++) cf[i] = (float)ct[i];
       QCHK(hipMemcpyAsync(ctx->Ct[sp], cf.data(), cnt * 4, hipMemcpyHostToDevice, ctx->stream));
+      QCHK(hipStreamSynchronize(ctx->stream));
+      // four consecutive functions of an orbital together, for the walk's rows
+      // (both spins as wide as the alpha spin's padded orbitals)
+      const size_t np = ctx->npad[sp], wide = ctx->npad[0], cnw = (size_t)walk_kpad(ctx->kpad, 4) * wide;
+      std::vector<float> cw(cnw, 0.0f);
+      for (size_t b = 0; b < (size_t)ctx->kpad; b++)
+        for (size_t o2 = 0; o2 < std::min(np, wide); o2++)
+          cw[((b >> 2) * wide + o2) * 4 + (b & 3)] = cf[b * np + o2];
+      QCHK(dalloc(ctx, &ctx->Cw[sp], cnw));
+      QCHK(hipMemcpyAsync(ctx->Cw[sp], cw.data(), cnw * 4, hipMemcpyHostToDevice, ctx->stream));
       QCHK(hipStreamSynchronize(ctx->stream));
     }
   }
@@ -1142,6 +1183,7 @@ size_t plan_device_bytes(const qmcb_system *s, const qmcb_options *o) {
   for (int sp = 0; sp < 2; sp++) {
     npad[sp] = pad_orb((int)std::max(nact[sp], 1L));
     add(kpad * npad[sp], tx);
+    if (tx == 4) add(walk_kpad((int)kpad, 4) * npad[0], 4);  // the walk's copy
   }
   if (o->replace_cusps)
     for (int sp = 0; sp < 2; sp++) {
@@ -1534,6 +1576,99 @@ static qmcb_status main_wait_groups(qmcb_ctx *ctx, int G) {
   return QMCB_OK;
 }
 
+// Arguments of a run of `steps` single-electron steps from `first` (walk.hip);
+// the caller sets the DMC fields.  The observable samples of the run's
+// sweeps go to vrow, which no walk keeps anything in.
+static WalkArgs walk_args(qmcb_ctx *ctx, long first, int steps, double tau, int mode, int num) {
+  WalkArgs a{};
+  a.sys = ctx->dsys;
+  for (int sp = 0; sp < 2; sp++) {
+    a.s[sp] = slater_args(ctx, sp);
+    a.Ct[sp] = ctx->Ct[sp];
+    a.Cw[sp] = ctx->Cw[sp];
+    a.npad[sp] = ctx->npad[sp];
+    a.cusp[sp] = ctx->cuspd[sp];
+  }
+  a.N = ctx->N;
+  a.n_up = ctx->n[0];
+  a.nsteps = steps;
+  a.first_step = first;
+  a.seed = ctx->opt.seed;
+  a.kpad = walk_kpad(ctx->kpad, ctx->tx);
+  a.np = ctx->np_shell;
+  a.pade_mn = ctx->pade_mn;
+  a.pade_md = ctx->pade_md;
+  a.pade_one = ctx->pade_one ? 1 : 0;
+  a.has_cusp = ctx->cusp ? 1 : 0;
+  a.R = ctx->R;
+  a.U = ctx->U; a.Ux = ctx->Ux; a.Uxx = ctx->Uxx; a.Vee = ctx->Vee; a.Ven = ctx->Ven;
+  a.cur_el = ctx->cur_el;
+  a.v_nn = ctx->dsys.v_nn;
+  a.tau = tau;
+  a.drift_mod = ctx->opt.drift_mod;
+  a.mode = mode;
+  a.acc_el = ctx->acc_el; a.acc_el2 = ctx->acc_el2; a.acc_n = ctx->acc_n;
+  a.acc_prop_el = ctx->acc_prop_el;
+  a.weight = ctx->weight;
+  a.acc_w = ctx->acc_w;
+  a.walk.age = ctx->age;
+  a.walk.old_walker = ctx->opt.old_walker_acceptance;
+  a.obs = (double *)ctx->vrow;
+  a.obs_stride = num;
+  return a;
+}
+
+// sweeps whose samples one run can keep in vrow
+static int walk_sweeps(const qmcb_ctx *ctx, int num) {
+  const size_t bytes = (size_t)kComp * std::max(ctx->npad[0], ctx->npad[1]) * ctx->ldv * ctx->to;
+  return (int)std::min<size_t>(1 << 16, bytes / (24 * (size_t)std::max(num, 1)));
+}
+
+// Steps of the run from step `first`, at most `left`: up to the first step
+// after which a re-inversion falls (staggered_refresh), as many sweeps as
+// walk_sweeps allows, one step with kernel timing (per-step launches).
+static int walk_run_length(const qmcb_ctx *ctx, long first, long left, int num) {
+  if (ctx->timing) return 1;
+  const int sweeps = walk_sweeps(ctx, num), K = ctx->rplan_K, S = ctx->rplan_S;
+  long mos[2] = {ctx->moves_of_spin[0], ctx->moves_of_spin[1]};
+  int rows = 0;
+  long n = 0;
+  while (n < left && n < (1 << 20)) {
+    const int m = (int)((first + n) % ctx->N), sp = m < ctx->n[0] ? 0 : 1;
+    if (m == 0 && rows == sweeps) break;
+    rows += m == 0;
+    n++;
+    if (ctx->opt.refresh_interval > 0 && K > 0) {
+      const int c = (int)(mos[sp] % K), q = c / S;
+      if (c == std::min(q * S + S - 1, K - 1)) break;
+    }
+    mos[sp]++;
+  }
+  return (int)std::max<long>(n, 1);
+}
+
+// Whether the single-electron steps of `num` walkers run as walk_kernel runs.
+// FP32 operands and 33 to 64 electrons a spin: a workgroup takes a CU, so 256
+// walkers run at once, about 16 us a step, while step by step a batch's time
+// grows less than its size (120 electrons, us a step: 75 against 101 at 1000
+// walkers, 312 against 237 at 4000).  With FP32 operands both ways take a
+// walker through the same bits, so its path does not depend on the choice;
+// with FP64 operands they differ by rounding, and the choice is the system's
+// alone.
+constexpr int kWalkRounds64 = 4 * 256;
+static bool walk_runs(const qmcb_ctx *ctx, int num) {
+  return ctx->walk && (ctx->tx == 8 || ctx->n[0] <= 32 || num <= kWalkRounds64);
+}
+
+// the counts of moves_of_spin after a run: every step but its last (which the
+// caller counts after the re-inversion that may follow it)
+static void walk_count(qmcb_ctx *ctx, long first, int steps) {
+  for (int i = 0; i + 1 < steps; i++) {
+    const int m = (int)((first + i) % ctx->N);
+    ctx->moves_of_spin[m < ctx->n[0] ? 0 : 1]++;
+  }
+}
+
 static qmcb_status series_reserve(qmcb_ctx *ctx, int64_t first_step, int32_t n_steps,
                                   int64_t N = 0) {
   if (N <= 0) N = ctx->N;
@@ -1805,6 +1940,47 @@ qmcb_status qmcb_vmc_steps(qmcb_ctx *ctx, int32_t num, int64_t first_step, int32
       if (gs != QMCB_OK) return gs;
       gs = groups_wait_main(ctx, G);
       if (gs != QMCB_OK) return gs;
+    }
+    if (walk_runs(ctx, num)) {
+      // runs of steps, one launch each (per group), up to the next re-inversion
+      for (int s = 0; s < count;) {
+        const long step = step0 + s;
+        const int L = walk_run_length(ctx, step, count - s, num);
+        const long last = step + L - 1;
+        const int sp = (int)(last % ctx->N) < ctx->n[0] ? 0 : 1;
+        const int rows = (int)(last / ctx->N - (step + ctx->N - 1) / ctx->N + 1);
+        WalkArgs a = walk_args(ctx, step, L, tau, 1, num);
+        walk_count(ctx, step, L);
+        qmcb_status st = QMCB_OK;
+        for (int g = 0; g < G && st == QMCB_OK; g++) {
+          const long first = (long)num * g / G, cnt = (long)num * (g + 1) / G - first;
+          WalkArgs ag = a;
+          ag.obs += 3 * first;
+          if (G > 1) {
+            GroupView view(ctx, g, first, sp);
+            st = DISPATCH(ctx, walk(ctx, ag, ctx->d_iota + first, (int)cnt));
+            if (st == QMCB_OK) st = staggered_refresh(ctx, first, first + cnt, sp);
+          } else {
+            st = DISPATCH(ctx, walk(ctx, ag, nullptr, num));
+            if (st == QMCB_OK) st = staggered_refresh(ctx, 0, num, sp);
+          }
+        }
+        if (st != QMCB_OK) return st;
+        ctx->moves_of_spin[sp]++;
+        if (rows > 0) {
+          if (G > 1) st = main_wait_groups(ctx, G);
+          if (st != QMCB_OK) return st;
+          TIMED("series", launch_series_reduce((const double *)ctx->vrow, num,
+                                               ctx->d_series + 4L * ctx->series_len, ctx->stream,
+                                               rows));
+          ctx->series_len += rows;
+          if (G > 1) st = groups_wait_main(ctx, G);
+          if (st != QMCB_OK) return st;
+        }
+        s += L;
+      }
+      if (G > 1) return main_wait_groups(ctx, G);
+      return QMCB_OK;
     }
     for (int s = 0; s < count; s++) {
       const long step = step0 + s;
@@ -2168,7 +2344,18 @@ qmcb_status qmcb_dmc_steps(qmcb_ctx *ctx, int64_t first_step, int32_t n_steps,
     }
   }
   for (int s = 0; s < n_steps; s++) {
-    const long step = first_step + s;
+    long step = first_step + s;
+    int run_len = 1;
+    // runs of steps in one launch each
+    const bool runs = !ae && walk_runs(ctx, std::max((int)ctx->active.size(), 1));
+    if (runs) {
+      // up to the next branching (the move of electron 0) or re-inversion
+      const long to0 = (ctx->N - step % ctx->N) % ctx->N + 1;
+      const int pop_ = (int)ctx->active.size();
+      run_len = walk_run_length(ctx, step, std::min<long>(to0, n_steps - s), std::max(pop_, 1));
+      step += run_len - 1;  // the run's last step: below, `step` and m are its
+      s += run_len - 1;
+    }
     const int m = ae ? 0 : (int)(step % ctx->N);
     const int pop = (int)ctx->active.size();
     if (pop == 0) {
@@ -2179,10 +2366,27 @@ qmcb_status qmcb_dmc_steps(qmcb_ctx *ctx, int64_t first_step, int32_t n_steps,
     // the reference's iteration = step - equilibration_steps; the stricter
     // deletion rules hold while iteration < -100 (QMCWalker.cpp:1207)
     walk.equilibrating = step < (long)prm->equilibration_steps - 100 ? 1 : 0;
-    // one group's step over the active-list rows [first, first + cnt) (g < 0:
-    // no groups)
+    double *const obs_base = (double *)ctx->vrow;  // a GroupView moves ctx->vrow
+    // one group's step (or run of steps) over the active-list rows [first,
+    // first + cnt) (g < 0: no groups)
     auto group_step = [&](long first, int cnt, int g) -> qmcb_status {
       const int *d_map = ctx->d_active + first;
+      if (runs) {
+        WalkArgs a = walk_args(ctx, step - run_len + 1, run_len, prm->tau, 2, pop);
+        a.obs = obs_base + 3 * first;
+        a.e_trial = ctx->e_trial;
+        a.e_est = ctx->e_est;
+        a.energy_mod = prm->energy_modification;
+        a.tau_eff = prm->tau;
+        a.reweight = (m == 0 && step >= prm->reweight_after) ? 1 : 0;
+        a.walk.equilibrating = walk.equilibrating;
+        a.walk.rel_cutoff = walk.rel_cutoff;
+        a.walk.e_orig = walk.e_orig;
+        a.walk.branch_threshold = walk.branch_threshold;
+        qmcb_status wst = DISPATCH(ctx, walk(ctx, a, d_map, cnt));
+        if (wst != QMCB_OK) return wst;
+        return staggered_refresh(ctx, first, first + cnt, sp);
+      }
       ProposeArgs pa{};
       pa.N = ctx->N;
       pa.moved = m;
@@ -2238,6 +2442,7 @@ qmcb_status qmcb_dmc_steps(qmcb_ctx *ctx, int64_t first_step, int32_t n_steps,
     };
     const int Geff = (G > 1 && pop / G >= 256) ? G : 1;
     ctx->last_groups = Geff;
+    if (runs) walk_count(ctx, step - run_len + 1, run_len);
     qmcb_status sst = QMCB_OK;
     if (ae) {
       ae_a.step = step;
@@ -2251,7 +2456,7 @@ qmcb_status qmcb_dmc_steps(qmcb_ctx *ctx, int64_t first_step, int32_t n_steps,
       for (int g = 0; g < G; g++) {
         const long first = (long)pop * g / G, cnt = (long)pop * (g + 1) / G - first;
         GroupView view(ctx, g, first, sp);
-        if (g > 0) QCHK(hipStreamWaitEvent(ctx->stream, ctx->gfront[g - 1], 0));
+        if (g > 0 && !runs) QCHK(hipStreamWaitEvent(ctx->stream, ctx->gfront[g - 1], 0));
         sst = group_step(first, (int)cnt, g);
         if (sst != QMCB_OK) return sst;
       }
@@ -2263,9 +2468,9 @@ qmcb_status qmcb_dmc_steps(qmcb_ctx *ctx, int64_t first_step, int32_t n_steps,
     }
     if (!ae) ctx->moves_of_spin[sp]++;
     if (m == 0)
-      TIMED("series", launch_series_reduce(ctx->d_obs, pop, ctx->d_series + 4L * ctx->series_len++,
-                                           ctx->stream));
-    moves += pop;
+      TIMED("series", launch_series_reduce(runs ? (const double *)ctx->vrow : ctx->d_obs, pop,
+                                           ctx->d_series + 4L * ctx->series_len++, ctx->stream));
+    moves += (long)pop * run_len;
     if (m != 0) {
       if (G > 1) {
         // the groups of the next step start after everything queued so far

@@ -8,6 +8,7 @@
 #include <type_traits>
 
 #include "qmcb_common.hpp"
+#include "qmcb_cusp.hpp"
 
 namespace qmcb {
 
@@ -82,7 +83,6 @@ struct GemmOut {
 };
 
 // cusp replacement added to GEMM output rows (device tables in qmcb_cusp.hpp)
-struct CuspDev;
 template <typename TO>
 hipError_t launch_cusp(const CuspDev &c, const PointSet &pts, const GemmOut &o, hipStream_t st);
 
@@ -255,8 +255,10 @@ struct MoveArgs {
 };
 
 // One row {sum w E, sum w, sum w p, walkers} of the per-sweep observable
-// series from obs[3 * num] (single workgroup, fixed summation order).
-hipError_t launch_series_reduce(const double *obs, int num, double *row, hipStream_t st);
+// series from obs[3 * num] (one workgroup a row, fixed summation order); rows
+// consecutive samples obs[rows][num][3] make rows rows.
+hipError_t launch_series_reduce(const double *obs, int num, double *row, hipStream_t st,
+                                int rows = 1);
 
 // several determinants (multidet.hip): per-spin Slater records with ndet /
 // nact / occ set, staging per (batch row, determinant) at b * D + d
@@ -320,6 +322,43 @@ hipError_t launch_sm_move(const MoveArgs &a, const int *walkers, int num, hipStr
 // electrons when n electrons of the moved spin set its tile (one electron
 // per thread)
 bool sm_move_fuses_jastrow(int n, int N);
+
+// A run of nsteps single-electron moves of the device walk in one launch (one
+// determinant; walk.hip): step first_step + s moves electron (first_step + s)
+// mod N of every walker.
+struct WalkArgs {
+  DevSystem sys;
+  SlaterArgs s[2];
+  int N, n_up, nsteps;
+  long first_step;
+  uint64_t seed;
+  const void *Ct[2];     // coefficients [kpad][npad] in the operand type
+  const float *Cw[2];    // FP32 operands: the same as [kpad / 4][npad[0]][4]
+                         // (zero rows up to kpad, a multiple of 48 then)
+  int npad[2], kpad;
+  int np;                // primitives, each shell's counted once
+  int pade_mn, pade_md;  // most numerator / denominator terms of any Pade function
+  int pade_one;          // every one has exactly one of each
+  int has_cusp;
+  CuspDev cusp[2];
+  double *R, *U, *Ux, *Uxx, *Vee, *Ven, *cur_el;
+  double v_nn, tau;
+  int drift_mod;
+  int mode;              // 1 VMC, 2 DMC (fixed node, weights)
+  double *acc_el, *acc_el2, *acc_n, *acc_prop_el;
+  double *weight, *acc_w;
+  double e_trial, tau_eff, e_est;
+  int reweight;          // reweight at the steps that move electron 0
+  int energy_mod;
+  WalkCtl walk;
+  double *obs;           // [sweeps of the run][obs_stride][3] observable samples
+  long obs_stride;
+};
+template <typename TS, typename TX>
+hipError_t launch_walk(const WalkArgs &a, const int *walkers, int num, hipStream_t st);
+// whether a system's run fits the kernel's LDS (tx: bytes of the GEMM operand)
+// (np: primitives, each shell's counted once)
+bool walk_fits(int n_up, int B, int kpad, int nn, int nshell, int np, int mn, int md, size_t tx);
 
 // ---- kernel (d): Jastrow + Coulomb, all-electron and single-electron ----
 struct JastrowArgs {

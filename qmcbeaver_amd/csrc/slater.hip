@@ -1288,6 +1288,8 @@ __global__ void __launch_bounds__(1024)
 series_reduce_kernel(const double *obs, int num, double *row) {
   __shared__ double red[3][16];
   const int t = threadIdx.x;
+  obs += 3L * num * blockIdx.x;
+  row += 4L * blockIdx.x;
   double se = 0.0, sw = 0.0, sp = 0.0;
   for (int b = t; b < num; b += 1024) {
     const double e = obs[3L * b], w = obs[3L * b + 1], p = obs[3L * b + 2];
@@ -1312,8 +1314,9 @@ series_reduce_kernel(const double *obs, int num, double *row) {
   if (t == 3) row[3] = (double)num;
 }
 
-hipError_t launch_series_reduce(const double *obs, int num, double *row, hipStream_t st) {
-  hipLaunchKernelGGL(series_reduce_kernel, dim3(1), dim3(1024), 0, st, obs, num, row);
+hipError_t launch_series_reduce(const double *obs, int num, double *row, hipStream_t st, int rows) {
+  if (rows <= 0) return hipSuccess;
+  hipLaunchKernelGGL(series_reduce_kernel, dim3(rows), dim3(1024), 0, st, obs, num, row);
   return hipGetLastError();
 }
 
