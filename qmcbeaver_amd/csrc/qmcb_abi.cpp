@@ -132,6 +132,9 @@ struct qmcb_ctx {
   void *Ct[2] = {nullptr, nullptr};
   // device output arrays (batch rows) for the host-buffer entry points
   qmcb_results dout{};
+  // pinned host staging of the host-buffer entry points (pin_reserve)
+  char *pin = nullptr;
+  size_t pin_cap = 0;
   int *d_ids = nullptr;
   uint8_t *d_mask = nullptr;
   // vmc accumulators
@@ -170,7 +173,7 @@ struct qmcb_ctx {
   int staged_moved = -1;
   int staged_num = 0;
   std::vector<int> staged_ids;
-  std::map<int, int> staged_row;
+  std::vector<int> staged_row;  // [Wc] row of a staged slot, -1: not staged
   std::vector<int> initialized;  // per slot: has a resident state
   int auto_groups = 0;           // walker_groups < 0: the count chosen by timing (0: not yet)
   int auto_groups_num = 0;       // ... for this many walkers
@@ -1055,6 +1058,7 @@ qmcb_status create_impl(const qmcb_system *s, const qmcb_options *o, qmcb_ctx *c
   QCHK(dalloc(ctx, &r.mod_ratio, W));
   QCHK(dalloc(ctx, &r.r2, W * 3));
   ctx->initialized.assign(ctx->Wc, 0);
+  ctx->staged_row.assign(ctx->Wc, -1);
   QCHK(hipStreamSynchronize(ctx->stream));
   return QMCB_OK;
 }
@@ -1075,32 +1079,101 @@ qmcb_status ensure_staging(qmcb_ctx *ctx) {
   return QMCB_OK;
 }
 
+// Pinned host staging of at least `bytes` (null beyond kPinMax, where a copy's
+// own time hides its fixed cost, or where the host has none to pin).  A copy
+// to or from pageable memory waits for itself, about 12 us each; through the
+// staging a call's small copies are one, and its inputs none the host waits on
+// (256 walkers of 64 electrons, 8 staged moves with their accepts: 4.11 ms
+// copy by copy, 2.40 through the staging).
+// Every entry point that uses it synchronises the stream before it returns.
+constexpr size_t kPinMax = (size_t)4 << 20;
+char *pin_reserve(qmcb_ctx *ctx, size_t bytes) {
+  if (bytes > kPinMax) return nullptr;
+  if (bytes > ctx->pin_cap) {
+    if (ctx->pin) {
+      (void)hipStreamSynchronize(ctx->stream);  // a copy may still be reading it
+      (void)hipHostFree(ctx->pin);
+    }
+    ctx->pin = nullptr;
+    ctx->pin_cap = 0;
+    void *p = nullptr;
+    const size_t cap = std::min(kPinMax, (2 * bytes + 4095) / 4096 * 4096);
+    if (hipHostMalloc(&p, cap, hipHostMallocDefault) != hipSuccess) {
+      (void)hipGetLastError();
+      return nullptr;
+    }
+    ctx->pin = (char *)p;
+    ctx->pin_cap = cap;
+  }
+  return ctx->pin;
+}
+
+// The result arrays of `num` rows one after another in the arena's output
+// block, the per-electron ones last, so that one copy brings them to the
+// host; `end` is the block's used size.  False where the arrays were not
+// carved as one block.
+bool packed_results(const qmcb_ctx *ctx, int num, qmcb_results &r, size_t &end) {
+  const qmcb_results &d = ctx->dout;
+  const size_t W = ctx->Wc, N3 = (size_t)ctx->N * 3;
+  char *base = (char *)d.log_psi;
+  const size_t block = 10 * arena_round(8 * W) + 2 * arena_round(W) + 2 * arena_round(8 * W * N3) +
+                       arena_round(24 * W);
+  if (!base || (char *)d.r2 + arena_round(24 * W) - base != (long)block) return false;
+  size_t at = 0;
+  auto take = [&](auto *&p, size_t bytes) {
+    p = (std::remove_reference_t<decltype(p)>)(base + at);
+    at += (bytes + 7) / 8 * 8;
+  };
+  const size_t n = num;
+  take(r.log_psi, 8 * n); take(r.lap_ratio, 8 * n); take(r.e_local, 8 * n);
+  take(r.kinetic, 8 * n); take(r.potential, 8 * n); take(r.v_ne, 8 * n); take(r.v_ee, 8 * n);
+  take(r.det_ratio, 8 * n); take(r.jastrow_u, 8 * n); take(r.mod_ratio, 8 * n);
+  take(r.r2, 24 * n); take(r.sign_psi, n); take(r.singular, n);
+  take(r.grad_lnpsi, 8 * n * N3); take(r.mod_drift, 8 * n * N3);
+  end = at;
+  return at <= block;
+}
+
 template <typename T>
 hipError_t d2h(qmcb_ctx *ctx, T *host, const T *dev, size_t count) {
   if (!host || !dev || count == 0) return hipSuccess;
   return hipMemcpyAsync(host, dev, count * sizeof(T), hipMemcpyDeviceToHost, ctx->stream);
 }
 
-qmcb_status copy_out(qmcb_ctx *ctx, int num, qmcb_results *out) {
+// The results `d` of `num` rows (packed, `end` bytes in all: one copy; end = 0:
+// array by array) to the host arrays the caller asked for.
+qmcb_status copy_out(qmcb_ctx *ctx, int num, qmcb_results *out, const qmcb_results &d, size_t end) {
   if (!out) return QMCB_OK;
-  const size_t N3 = (size_t)ctx->N * 3;
-  const qmcb_results &d = ctx->dout;
-  QCHK(d2h(ctx, out->log_psi, d.log_psi, num));
-  QCHK(d2h(ctx, out->sign_psi, d.sign_psi, num));
-  QCHK(d2h(ctx, out->grad_lnpsi, d.grad_lnpsi, num * N3));
-  QCHK(d2h(ctx, out->mod_drift, d.mod_drift, num * N3));
-  QCHK(d2h(ctx, out->lap_ratio, d.lap_ratio, num));
-  QCHK(d2h(ctx, out->e_local, d.e_local, num));
-  QCHK(d2h(ctx, out->kinetic, d.kinetic, num));
-  QCHK(d2h(ctx, out->potential, d.potential, num));
-  QCHK(d2h(ctx, out->v_ne, d.v_ne, num));
-  QCHK(d2h(ctx, out->v_ee, d.v_ee, num));
-  QCHK(d2h(ctx, out->det_ratio, d.det_ratio, num));
-  QCHK(d2h(ctx, out->jastrow_u, d.jastrow_u, num));
-  QCHK(d2h(ctx, out->singular, d.singular, num));
-  QCHK(d2h(ctx, out->mod_ratio, d.mod_ratio, num));
-  QCHK(d2h(ctx, out->r2, d.r2, num * 3));
-  QCHK(hipStreamSynchronize(ctx->stream));
+  const size_t N3 = (size_t)ctx->N * 3, n = num;
+  const char *base = (const char *)d.log_psi;
+  // without the per-electron arrays where nobody asks for them
+  if (end && !out->grad_lnpsi && !out->mod_drift) end = (const char *)d.grad_lnpsi - base;
+  char *pin = end ? pin_reserve(ctx, end) : nullptr;
+  if (pin) {
+    QCHK(hipMemcpyAsync(pin, base, end, hipMemcpyDeviceToHost, ctx->stream));
+    QCHK(hipStreamSynchronize(ctx->stream));
+  }
+  auto get = [&](auto *host, const auto *dev, size_t count) -> hipError_t {
+    if (!pin) return d2h(ctx, host, dev, count);
+    if (host) std::memcpy(host, pin + ((const char *)dev - base), count * sizeof(*host));
+    return hipSuccess;
+  };
+  QCHK(get(out->log_psi, d.log_psi, n));
+  QCHK(get(out->sign_psi, d.sign_psi, n));
+  QCHK(get(out->grad_lnpsi, d.grad_lnpsi, n * N3));
+  QCHK(get(out->mod_drift, d.mod_drift, n * N3));
+  QCHK(get(out->lap_ratio, d.lap_ratio, n));
+  QCHK(get(out->e_local, d.e_local, n));
+  QCHK(get(out->kinetic, d.kinetic, n));
+  QCHK(get(out->potential, d.potential, n));
+  QCHK(get(out->v_ne, d.v_ne, n));
+  QCHK(get(out->v_ee, d.v_ee, n));
+  QCHK(get(out->det_ratio, d.det_ratio, n));
+  QCHK(get(out->jastrow_u, d.jastrow_u, n));
+  QCHK(get(out->singular, d.singular, n));
+  QCHK(get(out->mod_ratio, d.mod_ratio, n));
+  QCHK(get(out->r2, d.r2, n * 3));
+  if (!pin) QCHK(hipStreamSynchronize(ctx->stream));
   return QMCB_OK;
 }
 
@@ -1318,6 +1391,7 @@ void qmcb_destroy(qmcb_ctx *ctx) {
   (void)hipSetDevice(ctx->device);
   if (ctx->stream) (void)hipStreamSynchronize(ctx->stream);
   for (void *p : ctx->allocs) (void)hipFree(p);
+  if (ctx->pin) (void)hipHostFree(ctx->pin);
   for (hipEvent_t e : ctx->tm.pool) (void)hipEventDestroy(e);
   if (ctx->ae_graph) (void)hipGraphExecDestroy(ctx->ae_graph);
 
@@ -1352,30 +1426,54 @@ qmcb_status qmcb_evaluate(qmcb_ctx *ctx, int32_t num, const int32_t *ids, const 
         return QMCB_BAD_STATE;
       }
   }
-  QCHK(hipMemcpyAsync(ctx->d_ids, ids, sizeof(int) * num, hipMemcpyHostToDevice, ctx->stream));
+  qmcb_results dout = ctx->dout;
+  size_t end = 0;
+  if (!packed_results(ctx, num, dout, end)) { dout = ctx->dout; end = 0; }
+  // inputs through the staging where they fit: ids, then the positions read
+  const size_t nid = (sizeof(int) * num + 7) / 8 * 8;
+  const size_t nr = sizeof(double) * 3 * num * (whichE == -1 ? ctx->N : 1);
+  char *pin = pin_reserve(ctx, std::max(nid + nr, end <= kPinMax ? end : (size_t)0));
   std::vector<double> pr;  // must outlive the asynchronous copy below
-  if (whichE == -1) {
-    QCHK(hipMemcpyAsync(ctx->Rin, R, sizeof(double) * num * ctx->N * 3, hipMemcpyHostToDevice,
-                        ctx->stream));
-  } else {
-    pr.resize((size_t)num * 3);
-    for (int i = 0; i < num; i++)
-      for (int k = 0; k < 3; k++) pr[3 * i + k] = R[((size_t)i * ctx->N + whichE) * 3 + k];
-    QCHK(hipMemcpyAsync(ctx->propR, pr.data(), sizeof(double) * num * 3, hipMemcpyHostToDevice,
-                        ctx->stream));
+  const int32_t *hid = ids;
+  const double *hr = R;
+  if (pin) {
+    std::memcpy(pin, ids, sizeof(int) * num);
+    hid = (const int32_t *)pin;
   }
-  s = evaluate_core(ctx, num, ctx->d_ids, ctx->Rin, whichE, ctx->dout);
-  if (s != QMCB_OK) return s;
-  s = copy_out(ctx, num, out);
-  if (s != QMCB_OK) return s;
+  if (whichE == -1) {
+    if (pin) {
+      std::memcpy(pin + nid, R, nr);
+      hr = (const double *)(pin + nid);
+    }
+  } else {
+    double *dst = pin ? (double *)(pin + nid) : nullptr;
+    if (!dst) {
+      pr.resize((size_t)num * 3);
+      dst = pr.data();
+    }
+    for (int i = 0; i < num; i++)
+      for (int k = 0; k < 3; k++) dst[3 * i + k] = R[((size_t)i * ctx->N + whichE) * 3 + k];
+    hr = dst;
+  }
+  QCHK(hipMemcpyAsync(ctx->d_ids, hid, sizeof(int) * num, hipMemcpyHostToDevice, ctx->stream));
+  QCHK(hipMemcpyAsync(whichE == -1 ? ctx->Rin : ctx->propR, hr, nr, hipMemcpyHostToDevice,
+                      ctx->stream));
+  s = evaluate_core(ctx, num, ctx->d_ids, ctx->Rin, whichE, dout);
+  if (s == QMCB_OK) s = copy_out(ctx, num, out, dout, end);
+  if (s != QMCB_OK || !out) {
+    // the staging (and pr) may still be being read
+    const hipError_t e = hipStreamSynchronize(ctx->stream);
+    if (s != QMCB_OK) return s;
+    QCHK(e);
+  }
   if (whichE == -1) {
     for (int i = 0; i < num; i++) ctx->initialized[ids[i]] = 1;
     ctx->staged_moved = -1;
   } else {
+    for (int id : ctx->staged_ids) ctx->staged_row[id] = -1;
     ctx->staged_moved = whichE;
     ctx->staged_num = num;
     ctx->staged_ids.assign(ids, ids + num);
-    ctx->staged_row.clear();
     for (int i = 0; i < num; i++) ctx->staged_row[ids[i]] = i;
   }
   return QMCB_OK;
@@ -1442,19 +1540,28 @@ qmcb_status qmcb_accept(qmcb_ctx *ctx, int32_t num, const int32_t *ids, const ui
     return QMCB_BAD_STATE;
   }
   QCHK(hipSetDevice(ctx->device));
-  std::vector<uint8_t> rowmask(ctx->staged_num, 0);
+  const size_t nid = (sizeof(int) * ctx->staged_num + 7) / 8 * 8;
+  char *pin = pin_reserve(ctx, nid + ctx->staged_num);
+  std::vector<uint8_t> own;
+  if (!pin) own.resize(ctx->staged_num);
+  uint8_t *rowmask = pin ? (uint8_t *)pin + nid : own.data();
+  std::memset(rowmask, 0, ctx->staged_num);
   for (int i = 0; i < num; i++) {
-    auto it = ctx->staged_row.find(ids[i]);
-    if (it == ctx->staged_row.end()) {
+    const int row = ids[i] >= 0 && ids[i] < ctx->Wc ? ctx->staged_row[ids[i]] : -1;
+    if (row < 0) {
       ctx->err = "walker id was not part of the staged proposal";
       return QMCB_INVALID_ARG;
     }
-    rowmask[it->second] = mask[i] ? 1 : 0;
+    rowmask[row] = mask[i] ? 1 : 0;
   }
-  QCHK(hipMemcpyAsync(ctx->d_ids, ctx->staged_ids.data(), sizeof(int) * ctx->staged_num,
-                      hipMemcpyHostToDevice, ctx->stream));
-  QCHK(hipMemcpyAsync(ctx->d_mask, rowmask.data(), ctx->staged_num, hipMemcpyHostToDevice,
+  const int *hid = ctx->staged_ids.data();
+  if (pin) {
+    std::memcpy(pin, hid, sizeof(int) * ctx->staged_num);
+    hid = (const int *)pin;
+  }
+  QCHK(hipMemcpyAsync(ctx->d_ids, hid, sizeof(int) * ctx->staged_num, hipMemcpyHostToDevice,
                       ctx->stream));
+  QCHK(hipMemcpyAsync(ctx->d_mask, rowmask, ctx->staged_num, hipMemcpyHostToDevice, ctx->stream));
   qmcb_status s;
   if (ctx->multi) {
     s = DISPATCH(ctx, mdet_commit(ctx, ctx->d_ids, ctx->d_mask, ctx->staged_num,
@@ -1484,10 +1591,59 @@ qmcb_status qmcb_refresh(qmcb_ctx *ctx, int32_t num, const int32_t *ids) {
 qmcb_status qmcb_get_positions(qmcb_ctx *ctx, int32_t num, double *R) {
   if (!ctx || num < 0 || num > ctx->Wc || (num > 0 && !R)) return QMCB_INVALID_ARG;
   QCHK(hipSetDevice(ctx->device));
-  QCHK(hipMemcpyAsync(R, ctx->R, sizeof(double) * num * ctx->N * 3, hipMemcpyDeviceToHost,
+  const size_t bytes = sizeof(double) * num * ctx->N * 3;
+  char *pin = bytes ? pin_reserve(ctx, bytes) : nullptr;
+  QCHK(hipMemcpyAsync(pin ? (void *)pin : (void *)R, ctx->R, bytes, hipMemcpyDeviceToHost,
                       ctx->stream));
   QCHK(hipStreamSynchronize(ctx->stream));
+  if (pin) std::memcpy(R, pin, bytes);
   return QMCB_OK;
+}
+
+// The energy accumulators are four arrays one after another in the arena
+// (acc_stride doubles apart): zeroed by one fill and read by one copy.
+static size_t acc_stride(const qmcb_ctx *ctx) { return arena_round(8 * (size_t)ctx->Wc) / 8; }
+static bool acc_block(const qmcb_ctx *ctx) {
+  const size_t s = acc_stride(ctx);
+  return ctx->acc_el2 == ctx->acc_el + s && ctx->acc_n == ctx->acc_el + 2 * s &&
+         ctx->acc_prop_el == ctx->acc_el + 3 * s;
+}
+static hipError_t zero_acc(qmcb_ctx *ctx, int num, bool weights) {
+  hipError_t e = hipSuccess;
+  if (acc_block(ctx)) {
+    e = hipMemsetAsync(ctx->acc_el, 0, 8 * (3 * acc_stride(ctx) + num), ctx->stream);
+  } else {
+    for (double *p : {ctx->acc_el, ctx->acc_el2, ctx->acc_n, ctx->acc_prop_el})
+      if (e == hipSuccess) e = hipMemsetAsync(p, 0, sizeof(double) * num, ctx->stream);
+  }
+  if (e == hipSuccess && weights)
+    e = hipMemsetAsync(ctx->acc_w, 0, sizeof(double) * num, ctx->stream);
+  return e;
+}
+// the sums of slots [0, num) on the host (in the staging or in `own`), the
+// stream synchronised
+static hipError_t get_acc(qmcb_ctx *ctx, int num, std::vector<double> &own, const double *&el,
+                          const double *&el2, const double *&n, const double *&prop) {
+  const size_t s = acc_stride(ctx), all = 3 * s + num;
+  double *h = (double *)pin_reserve(ctx, 8 * all);
+  if (!h) {
+    own.resize(all);
+    h = own.data();
+  }
+  hipError_t e = hipSuccess;
+  if (acc_block(ctx)) {
+    e = hipMemcpyAsync(h, ctx->acc_el, 8 * all, hipMemcpyDeviceToHost, ctx->stream);
+  } else {
+    const double *src[4] = {ctx->acc_el, ctx->acc_el2, ctx->acc_n, ctx->acc_prop_el};
+    for (int i = 0; i < 4 && e == hipSuccess; i++)
+      e = hipMemcpyAsync(h + i * s, src[i], 8 * (size_t)num, hipMemcpyDeviceToHost, ctx->stream);
+  }
+  if (e == hipSuccess) e = hipStreamSynchronize(ctx->stream);
+  el = h;
+  el2 = h + s;
+  n = h + 2 * s;
+  prop = h + 3 * s;
+  return e;
 }
 
 // Rows of the observable series a step range records: one per step that
@@ -1865,10 +2021,7 @@ qmcb_status qmcb_vmc_steps(qmcb_ctx *ctx, int32_t num, int64_t first_step, int32
       return QMCB_BAD_STATE;
     }
   QCHK(hipSetDevice(ctx->device));
-  QCHK(hipMemsetAsync(ctx->acc_el, 0, sizeof(double) * num, ctx->stream));
-  QCHK(hipMemsetAsync(ctx->acc_el2, 0, sizeof(double) * num, ctx->stream));
-  QCHK(hipMemsetAsync(ctx->acc_n, 0, sizeof(double) * num, ctx->stream));
-  QCHK(hipMemsetAsync(ctx->acc_prop_el, 0, sizeof(double) * num, ctx->stream));
+  QCHK(zero_acc(ctx, num, false));
   const bool ae = ctx->opt.all_electron_moves != 0;
   {
     qmcb_status rs = series_reserve(ctx, first_step, n_steps, ae ? 1 : 0);
@@ -2167,12 +2320,9 @@ qmcb_status qmcb_vmc_steps(qmcb_ctx *ctx, int32_t num, int64_t first_step, int32
     if (rs != QMCB_OK) return rs;
   }
   if (stats) {
-    std::vector<double> a(num), b(num), c(num), d(num);
-    QCHK(hipMemcpyAsync(a.data(), ctx->acc_el, sizeof(double) * num, hipMemcpyDeviceToHost, ctx->stream));
-    QCHK(hipMemcpyAsync(b.data(), ctx->acc_el2, sizeof(double) * num, hipMemcpyDeviceToHost, ctx->stream));
-    QCHK(hipMemcpyAsync(c.data(), ctx->acc_n, sizeof(double) * num, hipMemcpyDeviceToHost, ctx->stream));
-    QCHK(hipMemcpyAsync(d.data(), ctx->acc_prop_el, sizeof(double) * num, hipMemcpyDeviceToHost, ctx->stream));
-    QCHK(hipStreamSynchronize(ctx->stream));
+    std::vector<double> own;
+    const double *a, *b, *c, *d;
+    QCHK(get_acc(ctx, num, own, a, b, c, d));
     stats->sum_e_local = stats->sum_e_local_sq = stats->sum_accept = stats->sum_prop_e_local = 0;
     for (int i = 0; i < num; i++) {
       stats->sum_e_local += a[i];
@@ -2268,11 +2418,7 @@ qmcb_status qmcb_dmc_steps(qmcb_ctx *ctx, int64_t first_step, int32_t n_steps,
   }
   QCHK(hipSetDevice(ctx->device));
   const int W = ctx->Wc;
-  QCHK(hipMemsetAsync(ctx->acc_el, 0, sizeof(double) * W, ctx->stream));
-  QCHK(hipMemsetAsync(ctx->acc_el2, 0, sizeof(double) * W, ctx->stream));
-  QCHK(hipMemsetAsync(ctx->acc_n, 0, sizeof(double) * W, ctx->stream));
-  QCHK(hipMemsetAsync(ctx->acc_prop_el, 0, sizeof(double) * W, ctx->stream));
-  QCHK(hipMemsetAsync(ctx->acc_w, 0, sizeof(double) * W, ctx->stream));
+  QCHK(zero_acc(ctx, W, true));
   if (!ctx->have_e_trial) {
     // energy_estimated and energy_estimated_original start at the trial
     // energy (QMCFlags.cpp:918-919)
@@ -2587,13 +2733,11 @@ qmcb_status qmcb_dmc_steps(qmcb_ctx *ctx, int64_t first_step, int32_t n_steps,
   }
   // statistics
   {
-    std::vector<double> a(W), b2(W), c(W), d(W), wv(W);
-    QCHK(hipMemcpyAsync(a.data(), ctx->acc_el, sizeof(double) * W, hipMemcpyDeviceToHost, ctx->stream));
-    QCHK(hipMemcpyAsync(b2.data(), ctx->acc_el2, sizeof(double) * W, hipMemcpyDeviceToHost, ctx->stream));
-    QCHK(hipMemcpyAsync(c.data(), ctx->acc_n, sizeof(double) * W, hipMemcpyDeviceToHost, ctx->stream));
+    std::vector<double> own, d(W), wv(W);
+    const double *a, *b2, *c, *prop;
     QCHK(hipMemcpyAsync(d.data(), ctx->acc_w, sizeof(double) * W, hipMemcpyDeviceToHost, ctx->stream));
     QCHK(hipMemcpyAsync(wv.data(), ctx->weight, sizeof(double) * W, hipMemcpyDeviceToHost, ctx->stream));
-    QCHK(hipStreamSynchronize(ctx->stream));
+    QCHK(get_acc(ctx, W, own, a, b2, c, prop));  // synchronises
     for (int i = 0; i < W; i++) {
       st.sum_w_e_local += a[i];
       st.sum_w_e_local_sq += b2[i];
@@ -2633,11 +2777,13 @@ qmcb_status qmcb_sample_series(qmcb_ctx *ctx, int32_t cap, double *rows, int32_t
   QCHK(hipSetDevice(ctx->device));
   if (count) *count = ctx->series_len;
   const int n = std::min(cap, ctx->series_len);
+  char *pin = n > 0 ? pin_reserve(ctx, sizeof(double) * 4 * n) : nullptr;
   if (n > 0) {
-    QCHK(hipMemcpyAsync(rows, ctx->d_series, sizeof(double) * 4 * n, hipMemcpyDeviceToHost,
-                        ctx->stream));
+    QCHK(hipMemcpyAsync(pin ? (void *)pin : (void *)rows, ctx->d_series, sizeof(double) * 4 * n,
+                        hipMemcpyDeviceToHost, ctx->stream));
   }
   QCHK(hipStreamSynchronize(ctx->stream));
+  if (pin) std::memcpy(rows, pin, sizeof(double) * 4 * n);
   return QMCB_OK;
 }
 
