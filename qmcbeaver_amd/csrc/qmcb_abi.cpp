@@ -135,6 +135,7 @@ struct qmcb_ctx {
   // pinned host staging of the host-buffer entry points (pin_reserve)
   char *pin = nullptr;
   size_t pin_cap = 0;
+  bool orbitals_fit = true;  // every chunk of functions fits the fused orbital kernel
   int *d_ids = nullptr;
   uint8_t *d_mask = nullptr;
   // vmc accumulators
@@ -450,11 +451,29 @@ static bool jastrow_fused(const qmcb_ctx *ctx, int m) {
 // TS: derivative storage, TX: basis/GEMM operand, TO: GEMM output
 template <typename TS, typename TX, typename TC, typename TO>
 struct Engine {
+  // Basis functions and contraction in one kernel: every operand type but BF16
+  // (whose instruction takes 32 functions at once from an orbital-major copy),
+  // unless the environment fixes the tile of the separate contraction or a
+  // chunk's primitives exceed the kernel's LDS.
+  static bool orbitals_fused(const qmcb_ctx *ctx, long P, int sp) {
+    return sizeof(TX) >= 4 && ctx->orbitals_fit && !ctx->gemm_force.first &&
+           orbitals_workgroups(P, ctx->nact[sp]) <= kOrbWorkgroups;
+  }
+  template <typename T>
+  static qmcb_status orbitals(qmcb_ctx *ctx, const PointSet &pts, int sp, const GemmOut &go) {
+    if constexpr (sizeof(TX) >= 4)
+      TIMED("orbitals", (launch_orbitals<TX, T>(ctx->dsys, pts, (const TX *)ctx->Ct[sp],
+                                                ctx->npad[sp], ctx->nact[sp], ctx->kpad, go,
+                                                ctx->stream)));
+    return QMCB_OK;
+  }
+
   // all-electron: slots given by d_map (device) for batch rows [0, num); the
   // basis values go to X with a point capacity of ldp (the context's own
   // scratch unless the caller brings one)
   static qmcb_status all_electron(qmcb_ctx *ctx, const int *d_map, int num, void *Xs = nullptr,
                                   long ldp = 0) {
+    const bool own = !Xs;
     if (!Xs) {
       Xs = ctx->X;
       ldp = ctx->ldp;
@@ -462,7 +481,8 @@ struct Engine {
     for (int sp = 0; sp < 2; sp++) {
       const int n = ctx->n[sp];
       if (n == 0) continue;
-      const int chunk = std::max<long>(1, std::min<long>(num, ldp / n));
+      const bool fused = own && orbitals_fused(ctx, (long)num * n, sp);
+      const int chunk = fused ? num : std::max<long>(1, std::min<long>(num, ldp / n));
       if (!d_map && chunk < num) {
         ctx->err = "all-electron evaluate in chunks needs a walker map";
         return QMCB_INVALID_ARG;
@@ -471,18 +491,23 @@ struct Engine {
         const int cw = std::min(chunk, num - c0);
         PointSet pts{ctx->R + 3L * ctx->start[sp], (long)cw * n, n, 3L * ctx->N, 3,
                      d_map + c0};
-        TIMED("basis", (launch_basis<TC, TX>(ctx->dsys, pts, (TX *)Xs, ctx->kpad, ldp,
-                                            ctx->stream)));
         const long na = ctx->nact[sp];
         // derivative components at dm_at<TS>(k, o * n + e, na * n); values FP64 (o, e)
         const long e_s = dm_at<TS>(0, 1, 0), o_s = (long)n * e_s, k_s = dm_at<TS>(1, 0, na * n);
         GemmOut go{ctx->dmat[sp], k_s, o_s, (long)kDer * na * n, e_s, n, d_map + c0,
                    ctx->dval[sp], na * n, (long)n, 1};
-        TIMED("orbital_gemm", (launch_orbital_gemm<TX, TS>((const TX *)ctx->Ct[sp], ctx->npad[sp],
-                                                          (int)na,
-                                                          (const TX *)Xs, ctx->kpad, ldp,
-                                                          (long)cw * n, ctx->kpad, go,
-                                                          ctx->stream)));
+        if (fused) {
+          qmcb_status os = orbitals<TS>(ctx, pts, sp, go);
+          if (os != QMCB_OK) return os;
+        } else {
+          TIMED("basis", (launch_basis<TC, TX>(ctx->dsys, pts, (TX *)Xs, ctx->kpad, ldp,
+                                              ctx->stream)));
+          TIMED("orbital_gemm", (launch_orbital_gemm<TX, TS>((const TX *)ctx->Ct[sp],
+                                                            ctx->npad[sp], (int)na,
+                                                            (const TX *)Xs, ctx->kpad, ldp,
+                                                            (long)cw * n, ctx->kpad, go,
+                                                            ctx->stream)));
+        }
         if (ctx->cusp)
           TIMED("cusp", (launch_cusp<TS>(ctx->cuspd[sp], pts, go, ctx->stream)));
       }
@@ -539,11 +564,16 @@ struct Engine {
       TIMED("jastrow_move", launch_jastrow_move(ja, ctx->U, ctx->Ux, ctx->Uxx, ctx->Vee,
                                                 ctx->Ven, d_map, num, ctx->stream));
     PointSet pts{ctx->propR, (long)num, 1, 3, 0, nullptr};
-    TIMED("basis", (launch_basis<TC, TX>(ctx->dsys, pts, (TX *)ctx->X, ctx->kpad, ctx->ldp,
-                                        ctx->stream)));
-    const int n = ctx->n[sp];
     GemmOut go{ctx->vrow, (long)ctx->npad[sp], 1, (long)kComp * ctx->npad[sp], 0, 1, nullptr,
                nullptr, 0, 0, 0};
+    if (orbitals_fused(ctx, num, sp)) {
+      qmcb_status os = orbitals<TO>(ctx, pts, sp, go);
+      if (os != QMCB_OK) return os;
+      if (ctx->cusp) TIMED("cusp", (launch_cusp<TO>(ctx->cuspd[sp], pts, go, ctx->stream)));
+      return QMCB_OK;
+    }
+    TIMED("basis", (launch_basis<TC, TX>(ctx->dsys, pts, (TX *)ctx->X, ctx->kpad, ctx->ldp,
+                                        ctx->stream)));
     auto gemm = [&](std::pair<int, int> tile) {
       return launch_orbital_gemm<TX, TO>((const TX *)ctx->Ct[sp], ctx->npad[sp], ctx->nact[sp],
                                          (const TX *)ctx->X, ctx->kpad, ctx->ldp, (long)num,
@@ -556,7 +586,6 @@ struct Engine {
       it = ctx->gemm_tile.find(std::make_pair(sp, num >> 4));
     }
     TIMED("orbital_gemm", gemm(it->second));
-    (void)n;
     if (ctx->cusp) TIMED("cusp", (launch_cusp<TO>(ctx->cuspd[sp], pts, go, ctx->stream)));
     return QMCB_OK;
   }
@@ -834,6 +863,37 @@ qmcb_status create_impl(const qmcb_system *s, const qmcb_options *o, qmcb_ctx *c
     beg.push_back(ctx->nshell);
     d.nchunk = (int)beg.size() - 1;
     QCHK(upload(ctx, &d.chunk_beg, beg.data(), beg.size()));
+  }
+  {
+    // the fused orbital kernel's records
+    const int ns = ctx->nshell, nkc = (ctx->B + kOrbChunk - 1) / kOrbChunk;
+    ctx->orbitals_fit = nkc <= kOrbChunks;
+    std::vector<OrbShell> os(ns);
+    std::vector<OrbFn> of((size_t)nkc * kOrbChunk, OrbFn{{0, 0, 0}, 0, 0});
+    std::vector<int4> kc(nkc, int4{ns, 0, 0, 0});
+    std::vector<OrbPrim> pr;
+    for (int i = 0; i < ns; i++) {
+      OrbShell &q = os[i];
+      const double *x = s->nuc_xyz + 3 * sh.atom[i];
+      q = OrbShell{(int)pr.size(), sh.nprim[i], {0, 0}};
+      for (int j = sh.prim_off[i]; j < sh.prim_off[i] + q.np; j++)
+        pr.push_back(OrbPrim{{x[0], x[1], x[2]}, s->prim_alpha[j], s->prim_coef[j], 0.0});
+      const int f0 = sh.bf0[i], f1 = f0 + sh.ncart[i];
+      for (int c = f0 / kOrbChunk; c <= (f1 - 1) / kOrbChunk; c++) {
+        if (kc[c].x > i) kc[c].x = i, kc[c].z = q.p0;
+        kc[c].y = i + 1 - kc[c].x;
+        kc[c].w = q.p0 + q.np - kc[c].z;
+        if (kc[c].w > kOrbPrims) ctx->orbitals_fit = false;
+      }
+      for (int j = f0; j < f1; j++) {
+        of[j] = OrbFn{{x[0], x[1], x[2]}, i - kc[j / kOrbChunk].x, 0};
+        for (int k = 0; k < 3; k++) of[j].pw |= (s->bf_pow[3 * j + k] & 3) << (2 * k);
+      }
+    }
+    QCHK(upload(ctx, &d.orb_sh, os.data(), os.size()));
+    QCHK(upload(ctx, &d.orb_fn, of.data(), of.size()));
+    QCHK(upload(ctx, &d.orb_kc, kc.data(), kc.size()));
+    QCHK(upload(ctx, &d.orb_prim, pr.data(), pr.size()));
   }
   QCHK(upload(ctx, &d.prim_alpha, s->prim_alpha, (size_t)ctx->nprim));
   QCHK(upload(ctx, &d.prim_coef, s->prim_coef, (size_t)ctx->nprim));
@@ -1238,6 +1298,13 @@ size_t plan_device_bytes(const qmcb_system *s, const qmcb_options *o) {
   for (int i = 0; i < 5; i++) add(nshell, 4);
   add(3 * B, 4);
   add(std::max(1L, std::min(32L, nshell / 4)) + 1, 4);
+  const long nkc = (B + kOrbChunk - 1) / kOrbChunk;
+  long np_shell = 0;
+  for (int np : sh.nprim) np_shell += np;
+  add(nshell, sizeof(OrbShell));
+  add(nkc * kOrbChunk, sizeof(OrbFn));
+  add(nkc, sizeof(int4));
+  add(np_shell, sizeof(OrbPrim));
   add(s->n_prim, 8);
   add(s->n_prim, 8);
   add(nn, sizeof(qmcb_pade));

@@ -26,6 +26,23 @@ namespace qmcb {
 
 constexpr int kComp = 5;  // value, x, y, z, Laplacian
 
+// The records of the fused orbital kernel: a shell's primitives [p0, p0 + np)
+// of orb_prim; a primitive with its centre; a function's centre, powers (two
+// bits each for x, y, z) and shell, counted from the first of its chunk.
+struct OrbShell {
+  int p0, np, pad[2];
+};
+struct OrbPrim {
+  double c[3], alpha, coef, pad;
+};
+struct OrbFn {
+  double c[3];
+  int sh, pw;
+};
+constexpr int kOrbChunk = 32;    // basis functions formed and contracted at a time
+constexpr int kOrbPrims = 192;   // most primitives of a chunk's shells
+constexpr int kOrbChunks = 256;  // most chunks
+
 struct DevSystem {
   int N, n[2], start[2], nn, B, nshell, nprim;
   const double *nuc_xyz, *nuc_z;
@@ -33,6 +50,10 @@ struct DevSystem {
   const int *bf_pow;  // [B][3]
   const int *chunk_beg;  // [nchunk+1] shell ranges of the basis kernel's grid.y
   int nchunk;
+  const OrbShell *orb_sh;  // [nshell]
+  const OrbFn *orb_fn;     // [B rounded up to whole chunks]
+  const int4 *orb_kc;      // [chunks] first shell, shells, first primitive, primitives
+  const OrbPrim *orb_prim;  // primitives, shell by shell
   const double *prim_alpha, *prim_coef;
   qmcb_pade ee[3];                    // up-dn, up-up, dn-dn
   const qmcb_pade *en[2];             // [nn] per spin

@@ -92,6 +92,15 @@ hipError_t launch_scatter_rows(double *R, const double *Rin, const int *map, int
 // zero rows [B, ldk) of the five components of X[5][ldk][ldp] (elem bytes each)
 hipError_t launch_zero_pad_rows(void *X, size_t elem, int B, int ldk, long ldp, hipStream_t st);
 
+// ---- kernels (a) and (b) in one ----
+// `o`: the all-electron form (out_val, derivatives of an element together) or
+// rows of contiguous orbitals (s_orb 1, every orbital tile of 16 whole)
+long orbitals_workgroups(long P, int n_orb);
+constexpr long kOrbWorkgroups = 256;
+template <typename TX, typename TO>
+hipError_t launch_orbitals(const DevSystem &sys, const PointSet &pts, const TX *Ct, int ldc,
+                           int n_orb, int kpad, const GemmOut &o, hipStream_t st);
+
 // ---- kernel (a) ----
 template <typename TC, typename TS>
 hipError_t launch_basis(const DevSystem &sys, const PointSet &pts, TS *X, int ldk, long ldp,
