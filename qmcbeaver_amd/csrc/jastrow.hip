@@ -1,5 +1,7 @@
-// jastrow.hip -- kernel (d): two-body Pade Jastrow (e-e, e-n), Coulomb
-// potential and local-energy assembly, FP64.
+// jastrow.hip -- kernel (d): two-body Pade Jastrow (e-e, e-n) and Coulomb
+// potential of a single-electron move, local-energy assembly from the resident
+// state and the proposal of the step-by-step walk, FP64 (the all-electron
+// Jastrow is in finish.hip).
 //
 // Reference: QMCJastrow::evaluate (QMCJastrow.cpp:134-187),
 // QMCJastrowElectronElectron::updateAll/updateOne/collectForPair
@@ -37,70 +39,7 @@ __device__ __forceinline__ void block_sum(double *vals, int nv, double *scratch 
   __syncthreads();
 }
 
-// ---------------------------------------------------------------------------
-// all-electron Jastrow + potential, one workgroup per walker
 constexpr int kJT = 256;
-constexpr int kMaxN = 512;
-
-__global__ void __launch_bounds__(kJT) jastrow_all_kernel(JastrowArgs A, const int *walkers, int num) {
-  const int b = blockIdx.x;
-  if (b >= num) return;
-  const int w = walkers ? walkers[b] : b;
-  const DevSystem &S = A.sys;
-  const int N = S.N, nn = S.nn, nu = S.n[0];
-  __shared__ double x[kMaxN * 3];
-  __shared__ double scratch[4 * (kJT / 64)];
-  const double *Rw = A.R + (long)w * N * 3;
-  for (int i = threadIdx.x; i < 3 * N; i += kJT) x[i] = Rw[i];
-  __syncthreads();
-  double U = 0.0, Uxx = 0.0, Vee = 0.0, Ven = 0.0;
-  for (int i = threadIdx.x; i < N; i += kJT) {
-    double g[3] = {0.0, 0.0, 0.0};
-    const int sp = i < nu ? 0 : 1;
-    for (int A_ = 0; A_ < nn; A_++) {
-      double d[3], r2 = 0.0;
-      for (int k = 0; k < 3; k++) { d[k] = x[3 * i + k] - S.nuc_xyz[3 * A_ + k]; r2 += d[k] * d[k]; }
-      const double r = sqrt(r2), ir = 1.0 / r;
-      double u, du, d2u;
-      pade_eval(S.en[sp][A_], r, u, du, d2u);
-      U += u;
-      Uxx += 2.0 * ir * du + d2u;
-      for (int k = 0; k < 3; k++) g[k] += du * ir * d[k];
-      Ven -= S.nuc_z[A_] * ir;
-    }
-    for (int j = 0; j < N; j++) {
-      if (j == i) continue;
-      double d[3], r2 = 0.0;
-      for (int k = 0; k < 3; k++) { d[k] = x[3 * i + k] - x[3 * j + k]; r2 += d[k] * d[k]; }
-      const double r = sqrt(r2), ir = 1.0 / r;
-      double u, du, d2u;
-      pade_eval(S.ee[ee_type(i, j, nu)], r, u, du, d2u);
-      for (int k = 0; k < 3; k++) g[k] += du * ir * d[k];
-      if (j < i) {
-        U += u;
-        Uxx += 2.0 * (2.0 * ir * du + d2u);
-        Vee += ir;
-      }
-    }
-    double *ux = A.Ux + ((long)w * N + i) * 3;
-    ux[0] = g[0]; ux[1] = g[1]; ux[2] = g[2];
-  }
-  double v[4] = {U, Uxx, Vee, Ven};
-  block_sum<kJT>(v, 4, scratch);
-  if (threadIdx.x == 0) {
-    A.U[w] = v[0];
-    A.Uxx[w] = v[1];
-    A.Vee[w] = v[2];
-    A.Ven[w] = v[3];
-  }
-}
-
-hipError_t launch_jastrow_all(const JastrowArgs &a, const int *walkers, int num, hipStream_t st) {
-  if (num <= 0) return hipSuccess;
-  if (a.sys.N > kMaxN) return hipErrorInvalidValue;
-  hipLaunchKernelGGL(jastrow_all_kernel, dim3(num), dim3(kJT), 0, st, a, walkers, num);
-  return hipGetLastError();
-}
 
 // ---------------------------------------------------------------------------
 // single-electron Jastrow + potential at the proposal (updateOne,

@@ -471,8 +471,13 @@ struct Engine {
   // all-electron: slots given by d_map (device) for batch rows [0, num); the
   // basis values go to X with a point capacity of ldp (the context's own
   // scratch unless the caller brings one)
-  static qmcb_status all_electron(qmcb_ctx *ctx, const int *d_map, int num, void *Xs = nullptr,
-                                  long ldp = 0) {
+  // With the outputs `out` of assemble (same dt and what) and, where `ae` is
+  // given, the decision of that all-electron move and, if `propose`, the next
+  // step's proposal.
+  static qmcb_status all_electron(qmcb_ctx *ctx, const int *d_map, int num,
+                                  const qmcb_results &out, double dt = -1.0, int what = 3,
+                                  const AeArgs *ae = nullptr, bool propose = false,
+                                  void *Xs = nullptr, long ldp = 0) {
     const bool own = !Xs;
     if (!Xs) {
       Xs = ctx->X;
@@ -513,26 +518,36 @@ struct Engine {
       }
       SlaterArgs sa = slater_args(ctx, sp);
       TIMED("lu_inverse", launch_lu_inverse<TS>(sa, d_map, num, ctx->stream));
-      TIMED("traces_all", launch_traces_all<TS>(sa, d_map, num, ctx->stream));
+      if (ctx->multi) TIMED("traces_all", launch_traces_all<TS>(sa, d_map, num, ctx->stream));
+    }
+    if (!ctx->multi) {
+      FinishArgs f{};
+      f.a = assemble_args(ctx, out, dt, what);
+      f.U = ctx->U; f.Ux = ctx->Ux; f.Uxx = ctx->Uxx; f.Vee = ctx->Vee; f.Ven = ctx->Ven;
+      f.pade_one = ctx->pade_one ? 1 : 0;
+      f.move = ae ? 1 : 0;
+      f.propose = propose ? 1 : 0;
+      if (ae) f.ae = *ae;
+      TIMED("finish", launch_finish<TS>(f, d_map, num, ctx->stream));
+      return QMCB_OK;
     }
     JastrowArgs ja{};
     ja.sys = ctx->dsys;
     ja.R = ctx->R;
     ja.U = ctx->U; ja.Ux = ctx->Ux; ja.Uxx = ctx->Uxx; ja.Vee = ctx->Vee; ja.Ven = ctx->Ven;
-    TIMED("jastrow_all", launch_jastrow_all(ja, d_map, num, ctx->stream));
+    TIMED("jastrow_all", launch_jastrow_all(ja, ctx->pade_one, d_map, num, ctx->stream));
+    qmcb_status s = assemble(ctx, d_map, num, out, dt, what);
+    if (s != QMCB_OK || !ae) return s;
+    TIMED("ae_accept", launch_ae_accept(*ae, d_map, num, ctx->stream));
+    if (propose) {
+      AeArgs next = *ae;
+      next.step++;
+      TIMED("ae_propose", launch_ae_propose(next, d_map, num, ctx->stream));
+    }
     return QMCB_OK;
   }
 
-  // what: bit 0 writes each walker's current E_L (cur_el), bit 1 resets its
-  // age (a fresh walker); dt < 0: the context's time step for the drift
-  // modification
-  static qmcb_status assemble(qmcb_ctx *ctx, const int *d_map, int num, const qmcb_results &out,
-                              double dt = -1.0, int what = 3) {
-    if (ctx->multi) {
-      MdetArgs ma = mdet_args(ctx, -1, 0, out);
-      TIMED("mdet_assemble", launch_mdet_assemble(ma, d_map, num, ctx->stream));
-      return QMCB_OK;
-    }
+  static AssembleArgs assemble_args(qmcb_ctx *ctx, const qmcb_results &out, double dt, int what) {
     AssembleArgs aa{};
     aa.sys = ctx->dsys;
     aa.s[0] = slater_args(ctx, 0);
@@ -545,6 +560,20 @@ struct Engine {
     aa.out = out;
     aa.cur_el = (what & 1) ? ctx->cur_el : nullptr;
     aa.age = (what & 2) ? ctx->age : nullptr;
+    return aa;
+  }
+
+  // what: bit 0 writes each walker's current E_L (cur_el), bit 1 resets its
+  // age (a fresh walker); dt < 0: the context's time step for the drift
+  // modification
+  static qmcb_status assemble(qmcb_ctx *ctx, const int *d_map, int num, const qmcb_results &out,
+                              double dt = -1.0, int what = 3) {
+    if (ctx->multi) {
+      MdetArgs ma = mdet_args(ctx, -1, 0, out);
+      TIMED("mdet_assemble", launch_mdet_assemble(ma, d_map, num, ctx->stream));
+      return QMCB_OK;
+    }
+    const AssembleArgs aa = assemble_args(ctx, out, dt, what);
     TIMED("assemble", launch_assemble(aa, d_map, num, ctx->stream));
     return QMCB_OK;
   }
@@ -1253,9 +1282,7 @@ qmcb_status evaluate_core(qmcb_ctx *ctx, int num, const int *d_ids, const double
                           int whichE, const qmcb_results &dout) {
   if (whichE == -1) {
     QCHK(launch_scatter_rows(ctx->R, d_R, d_ids, num, ctx->N * 3, ctx->stream));
-    qmcb_status s = DISPATCH(ctx, all_electron(ctx, d_ids, num));
-    if (s != QMCB_OK) return s;
-    s = DISPATCH(ctx, assemble(ctx, d_ids, num, dout));
+    qmcb_status s = DISPATCH(ctx, all_electron(ctx, d_ids, num, dout));
     if (s != QMCB_OK) return s;
     return results_extra(ctx, num, d_ids, -1, dout);
   }
@@ -1593,9 +1620,8 @@ qmcb_status qmcb_evaluate_device_noalloc(qmcb_ctx *ctx, int32_t num, const int32
   QCHK(hipSetDevice(ctx->device));
   QCHK(launch_scatter_rows(ctx->R, R_dev, ids_dev, num, ctx->N * 3, ctx->stream));
   QCHK(launch_zero_pad_rows(ctx->scratch_dev, ctx->tx, ctx->B, ctx->kpad, cap, ctx->stream));
-  qmcb_status s = DISPATCH(ctx, all_electron(ctx, ids_dev, num, ctx->scratch_dev, cap));
-  if (s != QMCB_OK) return s;
-  s = DISPATCH(ctx, assemble(ctx, ids_dev, num, *out_dev));
+  qmcb_status s = DISPATCH(ctx, all_electron(ctx, ids_dev, num, *out_dev, -1.0, 3, nullptr, false,
+                                             ctx->scratch_dev, cap));
   if (s != QMCB_OK) return s;
   return results_extra(ctx, num, ids_dev, -1, *out_dev);
 }
@@ -2023,11 +2049,8 @@ static qmcb_status ae_begin(qmcb_ctx *ctx, const int *d_map, int num, const AeAr
 // measured no faster than the launches it holds).
 static qmcb_status ae_evaluate(qmcb_ctx *ctx, const int *d_map, int num, double tau) {
   auto eager = [&]() -> qmcb_status {
-    qmcb_status s = DISPATCH(ctx, all_electron(ctx, d_map, num));
-    if (s != QMCB_OK) return s;
-    return DISPATCH(ctx, assemble(ctx, d_map, num, ctx->dout, tau, 0));
+    return DISPATCH(ctx, all_electron(ctx, d_map, num, ctx->dout, tau, 0));
   };
-  if (ctx->timing || !ctx->opt.graphs) return eager();
   if (!(ctx->ae_graph && ctx->ae_graph_num == num && ctx->ae_graph_map == d_map &&
         ctx->ae_graph_tau == tau)) {
     const bool repeat = ctx->ae_last_num == num && ctx->ae_last_map == d_map &&
@@ -2063,18 +2086,28 @@ static qmcb_status ae_evaluate(qmcb_ctx *ctx, const int *d_map, int num, double 
   return QMCB_OK;
 }
 
-static qmcb_status ae_step(qmcb_ctx *ctx, const int *d_map, int num, const AeArgs &a) {
-  TIMED("ae_propose", launch_ae_propose(a, d_map, num, ctx->stream));
+// One move.  Without graphs its decision, and with `next` the proposal of the
+// step after it, ride in the evaluate's last kernel (drawn: this step's
+// proposal already was); a captured evaluate has no step-dependent argument, so
+// there they are launches of their own.
+static qmcb_status ae_step(qmcb_ctx *ctx, const int *d_map, int num, const AeArgs &a, bool drawn,
+                           bool next) {
+  if (!drawn) TIMED("ae_propose", launch_ae_propose(a, d_map, num, ctx->stream));
+  if (ctx->timing || !ctx->opt.graphs)
+    return DISPATCH(ctx, all_electron(ctx, d_map, num, ctx->dout, a.tau, 0, &a, next));
   const qmcb_status s = ae_evaluate(ctx, d_map, num, a.tau);
   if (s != QMCB_OK) return s;
   TIMED("ae_accept", launch_ae_accept(a, d_map, num, ctx->stream));
+  if (next) {
+    AeArgs an = a;
+    an.step++;
+    TIMED("ae_propose", launch_ae_propose(an, d_map, num, ctx->stream));
+  }
   return QMCB_OK;
 }
 
 static qmcb_status ae_end(qmcb_ctx *ctx, const int *d_map, int num) {
-  qmcb_status s = DISPATCH(ctx, all_electron(ctx, d_map, num));
-  if (s != QMCB_OK) return s;
-  return DISPATCH(ctx, assemble(ctx, d_map, num, ctx->dout, -1.0, 1));
+  return DISPATCH(ctx, all_electron(ctx, d_map, num, ctx->dout, -1.0, 1));
 }
 
 qmcb_status qmcb_vmc_steps(qmcb_ctx *ctx, int32_t num, int64_t first_step, int32_t n_steps,
@@ -2303,7 +2336,7 @@ qmcb_status qmcb_vmc_steps(qmcb_ctx *ctx, int32_t num, int64_t first_step, int32
     as = ae_begin(ctx, ctx->d_iota, num, a);
     for (int32_t i = 0; as == QMCB_OK && i < n_steps; i++) {
       a.step = first_step + i;
-      as = ae_step(ctx, ctx->d_iota, num, a);
+      as = ae_step(ctx, ctx->d_iota, num, a, i > 0, i + 1 < n_steps);
       if (as == QMCB_OK) {
         TIMED("series", launch_series_reduce(ctx->d_obs, num,
                                              ctx->d_series + 4L * ctx->series_len++, ctx->stream));
@@ -2663,7 +2696,7 @@ qmcb_status qmcb_dmc_steps(qmcb_ctx *ctx, int64_t first_step, int32_t n_steps,
       ae_a.e_trial = ctx->e_trial;
       ae_a.e_est = ctx->e_est;
       ae_a.walk = walk;
-      sst = ae_step(ctx, ctx->d_active, pop, ae_a);
+      sst = ae_step(ctx, ctx->d_active, pop, ae_a, false, false);
       if (sst != QMCB_OK) return sst;
     } else if (Geff > 1) {
       for (int g = 0; g < G; g++) {

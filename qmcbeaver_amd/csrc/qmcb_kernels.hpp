@@ -378,7 +378,9 @@ struct JastrowArgs {
   int moved;
   const double *propR;   // [Wc][3]
 };
-hipError_t launch_jastrow_all(const JastrowArgs &a, const int *walkers, int num, hipStream_t st);
+// pade_one: every Pade function has one numerator and one denominator term
+hipError_t launch_jastrow_all(const JastrowArgs &a, bool pade_one, const int *walkers, int num,
+                              hipStream_t st);
 hipError_t launch_jastrow_move(const JastrowArgs &a, const double *U, const double *Ux,
                                const double *Uxx, const double *Vee, const double *Ven,
                                const int *walkers, int num, hipStream_t st);
@@ -430,6 +432,20 @@ struct AeArgs {
 };
 hipError_t launch_ae_propose(const AeArgs &a, const int *walkers, int num, hipStream_t st);
 hipError_t launch_ae_accept(const AeArgs &a, const int *walkers, int num, hipStream_t st);
+
+// The end of a single-determinant all-electron evaluate: traces, Jastrow,
+// assembly (a's outputs; U, Ux, ... the resident Jastrow state written) and,
+// with `move`, the Metropolis decision `ae` of the proposal evaluated and, with
+// `propose`, the proposal of the step after it.
+struct FinishArgs {
+  AssembleArgs a;
+  double *U, *Ux, *Uxx, *Vee, *Ven;
+  int pade_one;
+  int move, propose;
+  AeArgs ae;
+};
+template <typename TS>
+hipError_t launch_finish(const FinishArgs &f, const int *walkers, int num, hipStream_t st);
 
 // commit staged single-electron proposals
 template <typename TS, typename TO>

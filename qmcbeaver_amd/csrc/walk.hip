@@ -49,6 +49,7 @@
 // registers) waits on each one, 130 cycles a read.
 #include "qmcb_cusp.hpp"
 #include "qmcb_kernels.hpp"
+#include "qmcb_pade.hpp"
 
 namespace qmcb {
 
@@ -95,58 +96,6 @@ __device__ __forceinline__ double quad_sum_own(double v0, double v1, double v2, 
   const bool hi = q & 2;
   const double keep = hi ? b : a, send = hi ? a : b;
   return keep + dpp_f64<0x4E>(send);
-}
-
-// Pade functions packed in LDS: {n_num, n_den as two ints}, num[mn], den[md]
-struct PadeShape {
-  int mn, md;
-  __host__ __device__ int stride() const { return 1 + mn + md; }
-};
-__device__ __forceinline__ void pade_general(const double *f, const PadeShape &ps, double r,
-                                              double &u, double &du, double &d2u) {
-  const long long cnt = __builtin_bit_cast(long long, f[0]);
-  const int nn = (int)cnt, nd = (int)(cnt >> 32);
-  const double *num = f + 1, *den = f + 1 + ps.mn;
-  double a = 0.0, ap = 0.0, app = 0.0;
-  if (nn > 0) {
-    a = num[nn - 1];
-    for (int i = nn - 2; i >= -1; i--) {
-      const double c = i >= 0 ? num[i] : 0.0;
-      app = app * r + ap;
-      ap = ap * r + a;
-      a = a * r + c;
-    }
-    app *= 2.0;
-  }
-  double b = 1.0, bp = 0.0, bpp = 0.0;
-  if (nd > 0) {
-    b = den[nd - 1];
-    for (int i = nd - 2; i >= -1; i--) {
-      const double c = i >= 0 ? den[i] : 1.0;
-      bpp = bpp * r + bp;
-      bp = bp * r + b;
-      b = b * r + c;
-    }
-    bpp *= 2.0;
-  }
-  const double ib = 1.0 / b;
-  u = a * ib;
-  du = (ap - u * bp) * ib;
-  d2u = (app - 2.0 * du * bp - u * bpp) * ib;
-}
-// u = a r / (1 + b r) (one term each), the same operations
-__device__ __forceinline__ void pade_first(const double *f, double r, double &u, double &du,
-                                           double &d2u) {
-  const double ap = f[1], bp = f[2];
-  const double b = __builtin_fma(bp, r, 1.0), ib = 1.0 / b;
-  u = ap * r * ib;
-  du = __builtin_fma(-u, bp, ap) * ib;
-  d2u = -(2.0 * du * bp) * ib;
-}
-__device__ __forceinline__ void pade_pack(double *dst, const PadeShape &ps, const qmcb_pade &f) {
-  dst[0] = __builtin_bit_cast(double, ((long long)f.n_den << 32) | (long long)(unsigned)f.n_num);
-  for (int i = 0; i < ps.mn; i++) dst[1 + i] = f.num[i];
-  for (int i = 0; i < ps.md; i++) dst[1 + ps.mn + i] = f.den[i];
 }
 
 // x^k by squaring (the walk's powers have whole exponents up to a few hundred)
@@ -653,7 +602,7 @@ walk_kernel(WalkArgs A, const int *walkers, int num) {
     if (64 * wave < max(N, nn)) {
       if (A.pade_one)
         jastrow([](const double *f, double x, double &u, double &du, double &d2u) {
-          pade_first(f, x, u, du, d2u);
+          pade_first(f + 1, x, u, du, d2u);
         });
       else
         jastrow([&](const double *f, double x, double &u, double &du, double &d2u) {
