@@ -516,10 +516,12 @@ struct Engine {
         if (ctx->cusp)
           TIMED("cusp", (launch_cusp<TS>(ctx->cuspd[sp], pts, go, ctx->stream)));
       }
-      SlaterArgs sa = slater_args(ctx, sp);
-      TIMED("lu_inverse", launch_lu_inverse<TS>(sa, d_map, num, ctx->stream));
-      if (ctx->multi) TIMED("traces_all", launch_traces_all<TS>(sa, d_map, num, ctx->stream));
     }
+    const SlaterArgs sa[2] = {slater_args(ctx, 0), slater_args(ctx, 1)};
+    TIMED("lu_inverse", launch_lu_inverse<TS>(sa[0], d_map, num, ctx->stream, &sa[1]));
+    if (ctx->multi)
+      for (int sp = 0; sp < 2; sp++)
+        TIMED("traces_all", launch_traces_all<TS>(sa[sp], d_map, num, ctx->stream));
     if (!ctx->multi) {
       FinishArgs f{};
       f.a = assemble_args(ctx, out, dt, what);

@@ -150,7 +150,8 @@ constexpr int kDelay = 8;
 constexpr int kDer = 4;  // stored derivative components
 
 template <typename TS>
-hipError_t launch_lu_inverse(const SlaterArgs &a, const int *walkers, int num, hipStream_t st);
+hipError_t launch_lu_inverse(const SlaterArgs &a, const int *walkers, int num, hipStream_t st,
+                             const SlaterArgs *other = nullptr);
 template <typename TS>
 hipError_t launch_traces_all(const SlaterArgs &a, const int *walkers, int num, hipStream_t st);
 

@@ -18,167 +18,126 @@ namespace qmcb {
 template <typename TS>
 __device__ __forceinline__ double ld(const TS *p) { return (double)*p; }
 
+// Orders LDS accesses of one wave across its lanes (a compiler barrier; the
+// LDS itself serves one wave's accesses in order).
+__device__ __forceinline__ void wave_lds_sync() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
 // ---------------------------------------------------------------------------
-// Batched inverse by Gauss-Jordan elimination with partial (row) pivoting,
-// register resident: G*G threads as a GxG grid, thread (tr, tc) owns the
-// cyclic block a[tr + G i][tc + G j], i, j < R (n <= G R).  Per pivot step
-// the G owners of the pivot column find the pivot with wavefront shuffles,
-// and only the pivot row and column pass through LDS (two barriers/step).  ln|det| and sign
-// are accumulated from the pivots and row swaps; the LU of the reference
-// (Crout, implicit scaling, long double sums) gives the same inverse and
-// determinant up to rounding.  Singular (an all-zero pivot column) sets the
-// walker's singular flag, as calcOK = false does (QMCSlater.cpp:675-683).
-template <typename TS, int R, int G>
-__global__ void __launch_bounds__(G * G)
-lu_inverse_kernel(SlaterArgs A, const int *walkers, int num) {
-  const int D = det_count(A), d = blockIdx.x % D;
-  const int b = blockIdx.x / D;
+// Batched inverse by Gauss-Jordan elimination with partial (row) pivoting for
+// n <= NP, NP 16 or 32: a wave a matrix, four in a workgroup, no workgroup
+// barrier.  Lane l holds row (electron) l % NP of NP / (64 / NP) columns
+// (orbitals), the column groups by l / NP.  A pivot step is one chain -- the
+// column to all groups by a lane permute, the largest by DPP, the pivot row
+// through LDS, its reciprocal -- so it is the latency of a step that counts,
+// and many matrices in flight: 700 matrices of 25, both spins' together,
+// 37 us where a workgroup a matrix with two barriers a step took 40 us a
+// spin.  No row is moved: rows are pivoted where they are, and the permutation
+// is undone when the result is written.  ln|det| and sign are accumulated from
+// the pivots and the permutation; the LU of the reference (Crout, implicit
+// scaling, long double sums) gives the same inverse and determinant up to
+// rounding.  Singular (an all-zero pivot column) sets the walker's singular
+// flag, as calcOK = false does (QMCSlater.cpp:675-683).
+template <int NP>
+__global__ void __launch_bounds__(256)
+lu_wave_kernel(SlaterArgs A0, SlaterArgs A1, const int *walkers, int num) {
+  constexpr int G = 64 / NP, C = NP / G;
+  __shared__ double st_[4][NP][NP + 1];
+  __shared__ double prow_[4][NP];
+  __shared__ int pv_[4][NP];
+  const SlaterArgs &A = blockIdx.y == 0 ? A0 : A1;
+  const int D = det_count(A), lane = threadIdx.x & 63;
+  const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int rec = blockIdx.x * 4 + wv, d = rec % D, b = rec / D;
   if (b >= num) return;
   const int w0 = walkers ? walkers[b] : b;
   const int w = w0 * D + d;  // this determinant's record
   const int n = A.n, nact = act_count(A);
-  const int tid = threadIdx.x;
-  // tid = tr + G tc: the G owners of one column are G consecutive lanes
-  const int tr = tid % G, tc = tid / G;
-  constexpr int M = G * R;
-  __shared__ double prow[M], krow[M];
-  __shared__ double fcol[2][M];
-  __shared__ int s_piv[2];
-  __shared__ double s_max[2];
-  __shared__ int ipiv[M];
-  __shared__ int dest[M];
-  __shared__ int cur[M];
+  const int r = lane % NP, grp = lane / NP;
+  double(*st)[NP + 1] = st_[wv];
+  double *prow = prow_[wv];
+  int *pv = pv_[wv];
 
   const double *dv = A.dval + (long)w0 * nact * n;  // value matrix, (o, e)
-  double a[R][R];
+  double a[C];
 #pragma unroll
-  for (int i = 0; i < R; i++)
-#pragma unroll
-    for (int j = 0; j < R; j++) {
-      const int gi = tr + G * i, gj = tc + G * j;  // gi: electron, gj: orbital
-      double v = (gi == gj) ? 1.0 : 0.0;
-      if (gi < n && gj < n) v = ld(dv + (long)occ_row(A, d, gj) * n + gi);
-      a[i][j] = v;
-    }
+  for (int j = 0; j < C; j++) {
+    const int c = grp * C + j;
+    a[j] = r < n && c < n ? dv[(long)occ_row(A, d, c) * n + r] : 0.0;
+  }
   // |det| kept as mantissa * 2^expo to stay in range
   double mant = 1.0, sgn = 1.0;
-  int expo = 0;
+  int expo = 0, kr = 0;  // kr: the step that pivoted this lane's row
+  uint32_t used = 0;     // rows pivoted
   bool sing = false;
-  for (int k = 0; k < n; k++) {
-    const int kj = k / G, kt = k % G, buf = k & 1;
-    // ---- pivot search in column k (rows >= k) by its 16 owner lanes
-    if (tc == kt) {
-      double best = -1.0;
-      int bi = 0x7fffffff;
 #pragma unroll
-      for (int i = 0; i < R; i++) {
-        const int gi = tr + G * i;
-        double aik = 0.0;
-#pragma unroll
-        for (int j = 0; j < R; j++) aik = (j == kj) ? a[i][j] : aik;
-        fcol[buf][gi] = aik;
-        if (gi >= k && gi < n) {
-          const double v = fabs(aik);
-          if (v > best) { best = v; bi = gi; }
+  for (int k = 0; k < NP; k++) {
+    if (k < n && !sing) {
+      constexpr int CC = C;
+      const int kg = k / CC, kj = k % CC;
+      const double f = __shfl(a[kj], kg * NP + r, 64);
+      // largest of the rows not yet pivoted, the lowest row among equals
+      const double v = fabs(f);
+      double best = r < n && !((used >> r) & 1) && v >= 0.0 ? v : -1.0;
+      int p = r;
+      row16_argmax(best, p);
+      const double b0 = readlane_f64(best, 0);
+      int q = __builtin_amdgcn_readlane(p, 0);
+      double top = b0;
+      if constexpr (NP == 32) {
+        const double b1 = readlane_f64(best, 16);
+        if (b1 > b0) {
+          top = b1;
+          q = __builtin_amdgcn_readlane(p, 16);
         }
       }
-      if constexpr (G == 16) {
-        row16_argmax(best, bi);  // the owners are one DPP row of 16 lanes
+      if (!(top > 0.0)) {
+        sing = true;
       } else {
+        if (r == q) {
 #pragma unroll
-        for (int off = G / 2; off >= 1; off >>= 1) {
-          const double ob = __shfl_xor(best, off, 64);
-          const int oi = __shfl_xor(bi, off, 64);
-          if (ob > best || (ob == best && oi < bi)) { best = ob; bi = oi; }
+          for (int j = 0; j < C; j++) prow[grp * C + j] = a[j];
+          kr = k;
         }
-      }
-      if (tr == 0) { s_piv[buf] = bi; s_max[buf] = best; }
-    }
-    __syncthreads();
-    if (!(s_max[buf] > 0.0)) { sing = true; break; }
-    const int p = s_piv[buf], pi = p / G;
-    if (tid == 0) ipiv[k] = p;
-    if (tr == p % G) {
+        if (lane == 0) pv[k] = q;
+        wave_lds_sync();
+        const double piv = readlane_f64(f, q);
+        if (piv < 0) sgn = -sgn;
+        if (__builtin_popcount(used >> q) & 1) sgn = -sgn;
+        used |= 1u << q;
+        int e2;
+        mant = frexp(mant * fabs(piv), &e2);
+        expo += e2;
+        const double ip = 1.0 / piv;
+        // the pivot row scaled, the other rows reduced (in place)
 #pragma unroll
-      for (int i = 0; i < R; i++)
-        if (i == pi) {
-#pragma unroll
-          for (int j = 0; j < R; j++) prow[tc + G * j] = a[i][j];
+        for (int j = 0; j < C; j++) {
+          const bool own = j == kj && grp == kg;  // column k itself
+          const double pr = own ? ip : prow[grp * C + j] * ip;
+          const double x = own ? -f * ip : __builtin_fma(-f, pr, a[j]);
+          a[j] = r == q ? pr : x;
         }
-    }
-    if (tr == kt && p != k) {
-#pragma unroll
-      for (int i = 0; i < R; i++)
-        if (i == kj) {
-#pragma unroll
-          for (int j = 0; j < R; j++) krow[tc + G * j] = a[i][j];
-        }
-    }
-    __syncthreads();
-    if (p != k) {
-      if (tr == kt) {
-#pragma unroll
-        for (int i = 0; i < R; i++)
-          if (i == kj) {
-#pragma unroll
-            for (int j = 0; j < R; j++) a[i][j] = prow[tc + G * j];
-          }
-      }
-      if (tr == p % G) {
-#pragma unroll
-        for (int i = 0; i < R; i++)
-          if (i == pi) {
-#pragma unroll
-            for (int j = 0; j < R; j++) a[i][j] = krow[tc + G * j];
-          }
-      }
-      sgn = -sgn;
-    }
-    const double piv = prow[k];
-    if (piv < 0) sgn = -sgn;
-    int e2;
-    mant = frexp(mant * fabs(piv), &e2);
-    expo += e2;
-    const double ip = 1.0 / piv;
-    // ---- elimination: row k scaled, other rows reduced (in-place Gauss-Jordan)
-#pragma unroll
-    for (int i = 0; i < R; i++) {
-      const int gi = tr + G * i;
-      // column-k entry of row gi after the interchange
-      const double f = (gi == p) ? fcol[buf][k] : fcol[buf][gi];
-#pragma unroll
-      for (int j = 0; j < R; j++) {
-        const int gj = tc + G * j;
-        const double pr = (gj == k) ? ip : prow[gj] * ip;
-        if (gi == k) a[i][j] = pr;
-        else a[i][j] = (gj == k) ? -f * ip : a[i][j] - f * pr;
+        wave_lds_sync();
       }
     }
   }
-  if (tid == 0) {
-    // undo the row interchanges as column interchanges, in reverse order
-    for (int c = 0; c < n; c++) dest[c] = c;
-    if (!sing) {
-      for (int c = 0; c < n; c++) cur[c] = c;
-      for (int k = n - 1; k >= 0; k--) {
-        const int q = ipiv[k];
-        if (q != k) { const int t = cur[k]; cur[k] = cur[q]; cur[q] = t; }
-      }
-      for (int c = 0; c < n; c++) dest[cur[c]] = c;
-    }
-  }
-  __syncthreads();
-  double *inv = A.inv + (long)w * n * n;
   if (!sing) {
+    double *inv = A.inv + (long)w * n * n;
+    if (r < n) {
 #pragma unroll
-    for (int i = 0; i < R; i++)
-#pragma unroll
-      for (int j = 0; j < R; j++) {
-        const int gi = tr + G * i, gj = tc + G * j;
-        if (gi < n && gj < n) inv[(long)gi * n + dest[gj]] = a[i][j];
+      for (int j = 0; j < C; j++) {
+        const int c = grp * C + j;
+        if (c < n) st[kr][pv[c]] = a[j];
       }
+    }
+    wave_lds_sync();
+    for (int i = grp; i < n; i += G)
+      if (r < n) inv[(long)i * n + r] = st[i][r];
   }
-  if (tid == 0) {
+  if (lane == 0) {
     A.logdet[w] = sing ? 0.0 : log(mant) + expo * 0.6931471805599453;
     A.sgn[w] = sing ? 0.0 : sgn;
     A.singular[w] = sing ? 1 : 0;
@@ -233,14 +192,6 @@ __device__ __forceinline__ uint32_t wave_max_u32(uint32_t v) {
   const uint32_t a = __builtin_amdgcn_readlane(v, 0), b = __builtin_amdgcn_readlane(v, 16);
   const uint32_t c = __builtin_amdgcn_readlane(v, 32), e = __builtin_amdgcn_readlane(v, 48);
   return max(max(a, b), max(c, e));
-}
-
-// Orders LDS accesses of one wave across its lanes (a compiler barrier; the
-// LDS itself serves one wave's accesses in order).
-__device__ __forceinline__ void wave_lds_sync() {
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-  __builtin_amdgcn_wave_barrier();
-  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
 template <typename TS, int NP>
@@ -562,14 +513,29 @@ gj_mfma_kernel(SlaterArgs A, const int *walkers, int num) {
   }
 }
 
+// Both spins of an all-electron evaluate in one launch where the same tile of
+// lu_wave_kernel serves them (a spin without electrons: one).
 template <typename TS>
-hipError_t launch_lu_inverse(const SlaterArgs &a, const int *walkers, int num, hipStream_t st) {
+hipError_t launch_lu_inverse(const SlaterArgs &a, const int *walkers, int num, hipStream_t st,
+                             const SlaterArgs *other) {
+  if (other && other->n > 0 && a.n > 0) {
+    const bool one = a.n <= 32 && other->n <= 32 && (a.n <= 16) == (other->n <= 16);
+    if (!one) {
+      const hipError_t e = launch_lu_inverse<TS>(a, walkers, num, st, nullptr);
+      return e != hipSuccess ? e : launch_lu_inverse<TS>(*other, walkers, num, st, nullptr);
+    }
+  } else if (other && a.n <= 0) {
+    return launch_lu_inverse<TS>(*other, walkers, num, st, nullptr);
+  }
   if (num <= 0 || a.n <= 0) return hipSuccess;
+  const bool two = other && other->n > 0;
   const unsigned g = (unsigned)num * (a.ndet > 1 ? a.ndet : 1);
   if (a.n <= 16)
-    hipLaunchKernelGGL((lu_inverse_kernel<TS, 1, 16>), dim3(g), dim3(256), 0, st, a, walkers, num);
+    hipLaunchKernelGGL((lu_wave_kernel<16>), dim3((g + 3) / 4, two ? 2 : 1), dim3(256), 0, st, a,
+                       two ? *other : a, walkers, num);
   else if (a.n <= 32)
-    hipLaunchKernelGGL((lu_inverse_kernel<TS, 2, 16>), dim3(g), dim3(256), 0, st, a, walkers, num);
+    hipLaunchKernelGGL((lu_wave_kernel<32>), dim3((g + 3) / 4, two ? 2 : 1), dim3(256), 0, st, a,
+                       two ? *other : a, walkers, num);
   else if (a.n <= 64)
     hipLaunchKernelGGL((gj_mfma_kernel<TS, 64>), dim3(g), dim3(256), 0, st, a, walkers, num);
   else if (a.n <= 128)
@@ -1441,11 +1407,14 @@ INST(float, float)
 INST(float, double)
 INST(bf16s, float)
 #undef INST
-template hipError_t launch_lu_inverse<double>(const SlaterArgs &, const int *, int, hipStream_t);
-template hipError_t launch_lu_inverse<float>(const SlaterArgs &, const int *, int, hipStream_t);
+template hipError_t launch_lu_inverse<double>(const SlaterArgs &, const int *, int, hipStream_t,
+                                                const SlaterArgs *);
+template hipError_t launch_lu_inverse<float>(const SlaterArgs &, const int *, int, hipStream_t,
+                                                const SlaterArgs *);
 template hipError_t launch_traces_all<double>(const SlaterArgs &, const int *, int, hipStream_t);
 template hipError_t launch_traces_all<float>(const SlaterArgs &, const int *, int, hipStream_t);
-template hipError_t launch_lu_inverse<bf16s>(const SlaterArgs &, const int *, int, hipStream_t);
+template hipError_t launch_lu_inverse<bf16s>(const SlaterArgs &, const int *, int, hipStream_t,
+                                                const SlaterArgs *);
 template hipError_t launch_traces_all<bf16s>(const SlaterArgs &, const int *, int, hipStream_t);
 
 }  // namespace qmcb
