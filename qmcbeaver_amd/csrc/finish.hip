@@ -74,7 +74,7 @@ __device__ __forceinline__ void jastrow_block(const DevSystem &S, JastrowLds &L,
   if (nn <= kNuc) load_en(0);
   auto dist2 = [](const double *a, const double *b) {
     const double dx = a[0] - b[0], dy = a[1] - b[1], dz = a[2] - b[2];
-    return __builtin_fma(dz, dz, __builtin_fma(dy, dy, dx * dx));
+    return __builtin_fma(dz, dz, __builtin_fma(dx, dx, dy * dy));
   };
   // one coordinate of rows [r0, r0 + nr) gains `nc` partners at px, the pair's
   // value at w[row * sr + partner * sc]
