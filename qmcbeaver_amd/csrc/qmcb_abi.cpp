@@ -455,16 +455,18 @@ struct Engine {
   // (whose instruction takes 32 functions at once from an orbital-major copy),
   // unless the environment fixes the tile of the separate contraction or a
   // chunk's primitives exceed the kernel's LDS.
-  static bool orbitals_fused(const qmcb_ctx *ctx, long P, int sp) {
+  // `others`: workgroups of the launch besides
+  static bool orbitals_fused(const qmcb_ctx *ctx, long P, int sp, long others = 0) {
     return sizeof(TX) >= 4 && ctx->orbitals_fit && !ctx->gemm_force.first &&
-           orbitals_workgroups(P, ctx->nact[sp]) <= kOrbWorkgroups;
+           orbitals_workgroups(P, ctx->nact[sp]) + others <= kOrbWorkgroups;
+  }
+  static OrbSide orb_side(const qmcb_ctx *ctx, const PointSet &pts, int sp, const GemmOut &go) {
+    return OrbSide{pts, ctx->Ct[sp], ctx->npad[sp], ctx->nact[sp], go};
   }
   template <typename T>
-  static qmcb_status orbitals(qmcb_ctx *ctx, const PointSet &pts, int sp, const GemmOut &go) {
+  static qmcb_status orbitals(qmcb_ctx *ctx, const OrbSide &s0, const OrbSide *s1 = nullptr) {
     if constexpr (sizeof(TX) >= 4)
-      TIMED("orbitals", (launch_orbitals<TX, T>(ctx->dsys, pts, (const TX *)ctx->Ct[sp],
-                                                ctx->npad[sp], ctx->nact[sp], ctx->kpad, go,
-                                                ctx->stream)));
+      TIMED("orbitals", (launch_orbitals<TX, T>(ctx->dsys, s0, s1, ctx->kpad, ctx->stream)));
     return QMCB_OK;
   }
 
@@ -483,6 +485,26 @@ struct Engine {
       Xs = ctx->X;
       ldp = ctx->ldp;
     }
+    // points, outputs and map of a spin's electrons of rows [c0, c0 + cw)
+    auto side = [&](int sp, int c0, int cw) {
+      const int n = ctx->n[sp];
+      PointSet pts{ctx->R + 3L * ctx->start[sp], (long)cw * n, n, 3L * ctx->N, 3, d_map + c0};
+      const long na = ctx->nact[sp];
+      // derivative components at dm_at<TS>(k, o * n + e, na * n); values FP64 (o, e)
+      const long e_s = dm_at<TS>(0, 1, 0), o_s = (long)n * e_s, k_s = dm_at<TS>(1, 0, na * n);
+      GemmOut go{ctx->dmat[sp], k_s, o_s, (long)kDer * na * n, e_s, n, d_map + c0,
+                 ctx->dval[sp], na * n, (long)n, 1};
+      return orb_side(ctx, pts, sp, go);
+    };
+    // both spins in one launch where they fit one together
+    const bool both =
+        own && num > 0 && ctx->n[1] > 0 && orbitals_fused(ctx, (long)num * ctx->n[0], 0,
+                       orbitals_workgroups((long)num * ctx->n[1], ctx->nact[1]));
+    if (both) {
+      const OrbSide s0 = side(0, 0, num), s1 = side(1, 0, num);
+      qmcb_status os = orbitals<TS>(ctx, s0, &s1);
+      if (os != QMCB_OK) return os;
+    }
     for (int sp = 0; sp < 2; sp++) {
       const int n = ctx->n[sp];
       if (n == 0) continue;
@@ -494,21 +516,19 @@ struct Engine {
       }
       for (int c0 = 0; c0 < num; c0 += chunk) {
         const int cw = std::min(chunk, num - c0);
-        PointSet pts{ctx->R + 3L * ctx->start[sp], (long)cw * n, n, 3L * ctx->N, 3,
-                     d_map + c0};
-        const long na = ctx->nact[sp];
-        // derivative components at dm_at<TS>(k, o * n + e, na * n); values FP64 (o, e)
-        const long e_s = dm_at<TS>(0, 1, 0), o_s = (long)n * e_s, k_s = dm_at<TS>(1, 0, na * n);
-        GemmOut go{ctx->dmat[sp], k_s, o_s, (long)kDer * na * n, e_s, n, d_map + c0,
-                   ctx->dval[sp], na * n, (long)n, 1};
-        if (fused) {
-          qmcb_status os = orbitals<TS>(ctx, pts, sp, go);
+        const OrbSide q = side(sp, c0, cw);
+        const PointSet &pts = q.pts;
+        const GemmOut &go = q.out;
+        if (both) {
+          // formed above
+        } else if (fused) {
+          qmcb_status os = orbitals<TS>(ctx, q);
           if (os != QMCB_OK) return os;
         } else {
           TIMED("basis", (launch_basis<TC, TX>(ctx->dsys, pts, (TX *)Xs, ctx->kpad, ldp,
                                               ctx->stream)));
           TIMED("orbital_gemm", (launch_orbital_gemm<TX, TS>((const TX *)ctx->Ct[sp],
-                                                            ctx->npad[sp], (int)na,
+                                                            ctx->npad[sp], ctx->nact[sp],
                                                             (const TX *)Xs, ctx->kpad, ldp,
                                                             (long)cw * n, ctx->kpad, go,
                                                             ctx->stream)));
@@ -598,7 +618,7 @@ struct Engine {
     GemmOut go{ctx->vrow, (long)ctx->npad[sp], 1, (long)kComp * ctx->npad[sp], 0, 1, nullptr,
                nullptr, 0, 0, 0};
     if (orbitals_fused(ctx, num, sp)) {
-      qmcb_status os = orbitals<TO>(ctx, pts, sp, go);
+      qmcb_status os = orbitals<TO>(ctx, orb_side(ctx, pts, sp, go));
       if (os != QMCB_OK) return os;
       if (ctx->cusp) TIMED("cusp", (launch_cusp<TO>(ctx->cuspd[sp], pts, go, ctx->stream)));
       return QMCB_OK;
@@ -2334,14 +2354,21 @@ qmcb_status qmcb_vmc_steps(qmcb_ctx *ctx, int32_t num, int64_t first_step, int32
     AeArgs a{};
     ae_args(ctx, a, tau);
     a.mode = 1;
-    a.obs = ctx->d_obs;
     as = ae_begin(ctx, ctx->d_iota, num, a);
+    // the samples of as many steps as the single-electron rows' buffer holds
+    // (no all-electron move reads it) are reduced together
+    const int cap = walk_sweeps(ctx, num);
+    int rows = 0;
     for (int32_t i = 0; as == QMCB_OK && i < n_steps; i++) {
       a.step = first_step + i;
+      a.obs = (double *)ctx->vrow + 3L * num * rows++;
       as = ae_step(ctx, ctx->d_iota, num, a, i > 0, i + 1 < n_steps);
-      if (as == QMCB_OK) {
-        TIMED("series", launch_series_reduce(ctx->d_obs, num,
-                                             ctx->d_series + 4L * ctx->series_len++, ctx->stream));
+      if (as == QMCB_OK && (rows == cap || i + 1 == n_steps)) {
+        TIMED("series", launch_series_reduce((const double *)ctx->vrow, num,
+                                             ctx->d_series + 4L * ctx->series_len, ctx->stream,
+                                             rows));
+        ctx->series_len += rows;
+        rows = 0;
       }
     }
     if (as == QMCB_OK) as = ae_end(ctx, ctx->d_iota, num);

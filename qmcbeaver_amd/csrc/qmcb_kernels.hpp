@@ -97,9 +97,16 @@ hipError_t launch_zero_pad_rows(void *X, size_t elem, int B, int ldk, long ldp, 
 // rows of contiguous orbitals (s_orb 1, every orbital tile of 16 whole)
 long orbitals_workgroups(long P, int n_orb);
 constexpr long kOrbWorkgroups = 256;
+struct OrbSide {
+  PointSet pts;
+  const void *Ct;  // coefficients, operand type
+  int ldc, n_orb;
+  GemmOut out;
+};
+// s1: a second side (the other spin) in the same launch, or null
 template <typename TX, typename TO>
-hipError_t launch_orbitals(const DevSystem &sys, const PointSet &pts, const TX *Ct, int ldc,
-                           int n_orb, int kpad, const GemmOut &o, hipStream_t st);
+hipError_t launch_orbitals(const DevSystem &sys, const OrbSide &s0, const OrbSide *s1, int kpad,
+                           hipStream_t st);
 
 // ---- kernel (a) ----
 template <typename TC, typename TS>
