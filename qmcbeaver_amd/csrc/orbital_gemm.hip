@@ -10,7 +10,7 @@
 // Ct = C^T ([basis][orbital], zero padded to the orbital tile widths and to
 // 32-multiples of basis functions; BF16 operands keep C orbital-major,
 // [orbital][basis], so a lane's eight k values of one orbital are one 16-byte
-// LDS read), X from kernel (a).  One wavefront owns a 16-point tile and MT
+// LDS read), X from kernel (a).  One wavefront owns PW 16-point tiles and MT
 // 16-orbital tiles; each k-step issues MT MFMA instructions: 16x16x4 for
 // FP64 (v_mfma_f64_16x16x4f64) and FP32 (v_mfma_f32_16x16x4f32) with lane l
 // supplying A[l%16][l/16] and B[l/16][l%16]; gfx950's 16x16x32 for BF16
@@ -41,7 +41,7 @@ struct GemmTile {
   static constexpr int PAD = sizeof(TI) == 8 ? 8 : 16;  // elements
 };
 
-template <typename TI, typename TO, int MT, int WPB>
+template <typename TI, typename TO, int MT, int WPB, int PW>
 __global__ void __launch_bounds__(64 * WPB)
 orbital_gemm_kernel(const TI *__restrict__ Ct, int ldc, int n_orb, const TI *__restrict__ X,
                     int ldk, long ldp, long P, int kpad, GemmOut o) {
@@ -59,14 +59,19 @@ orbital_gemm_kernel(const TI *__restrict__ Ct, int ldc, int n_orb, const TI *__r
   __shared__ TI cs[2][LR][LW];
   const int tid = threadIdx.x;
   const int lane = tid & 63, wave = tid >> 6;
-  const long p0 = ((long)blockIdx.x * WPB + wave) * 16;
+  // the components of a point tile on one XCD, one after another (workgroups go
+  // to the eight XCDs in turn): an element's derivatives, four components, are
+  // one store of the L2 they meet in
+  const int local = blockIdx.x >> 3, comp = local % kComp;
+  const long p0 = (((long)(local / kComp) * 8 + (blockIdx.x & 7)) * WPB + wave) * 16 * PW;
   const bool live = p0 < P;  // wave-uniform
-  const int comp = blockIdx.y;
-  const int o0 = blockIdx.z * OW;
+  const int o0 = blockIdx.y * OW;
   const int li = lane & 15, lk = lane >> 4;
-  acc_t acc[MT];
+  acc_t acc[PW][MT];
 #pragma unroll
-  for (int t = 0; t < MT; t++) acc[t] = acc_t{0, 0, 0, 0};
+  for (int q = 0; q < PW; q++)
+#pragma unroll
+    for (int t = 0; t < MT; t++) acc[q][t] = acc_t{0, 0, 0, 0};
 
   // cooperative chunk load: element e = (j * NT + tid) * VE of the KC x OW
   // tile (OW x KC for orbital-major BF16, whose rows are kpad long)
@@ -92,13 +97,15 @@ orbital_gemm_kernel(const TI *__restrict__ Ct, int ldc, int n_orb, const TI *__r
   const int nch = kpad / KC;
   // the point operand of the next chunk is loaded with the next coefficient
   // chunk, one chunk ahead of its MFMAs (its HBM latency overlaps them)
-  TI b[KC / 4], bn[KC / 4];
-  auto bload = [&](int k0, TI *dst) {
+  TI b[PW][KC / 4], bn[PW][KC / 4];
+  auto bload = [&](int k0, TI (*dst)[KC / 4]) {
     if (!live) return;
+#pragma unroll
+    for (int q = 0; q < PW; q++)
 #pragma unroll
     for (int s = 0; s < KC / KS; s++)
 #pragma unroll
-      for (int j = 0; j < KPL; j++) dst[s * KPL + j] = xp[(long)(k0 + KS * s + j) * ldp];
+      for (int j = 0; j < KPL; j++) dst[q][s * KPL + j] = xp[(long)(k0 + KS * s + j) * ldp + 16 * q];
   };
   gload(0);
   bload(0, b);
@@ -118,18 +125,23 @@ orbital_gemm_kernel(const TI *__restrict__ Ct, int ldc, int n_orb, const TI *__r
 #pragma unroll
           for (int t = 0; t < MT; t++) a[t] = cs[buf][4 * s + lk][16 * t + li];
 #pragma unroll
-          for (int t = 0; t < MT; t++) acc[t] = M::run(a[t], b[s], acc[t]);
+          for (int q = 0; q < PW; q++)
+#pragma unroll
+            for (int t = 0; t < MT; t++) acc[q][t] = M::run(a[t], b[q][s], acc[q][t]);
         }
       } else {
 #pragma unroll
         for (int s = 0; s < KC / KS; s++) {
-          b8v bv;
+          b8v bv[PW];
 #pragma unroll
-          for (int j = 0; j < KPL; j++) bv[j] = __builtin_bit_cast(__bf16, b[s * KPL + j]);
+          for (int q = 0; q < PW; q++)
+#pragma unroll
+            for (int j = 0; j < KPL; j++) bv[q][j] = __builtin_bit_cast(__bf16, b[q][s * KPL + j]);
 #pragma unroll
           for (int t = 0; t < MT; t++) {
             const b8v av = *(const b8v *)&cs[buf][16 * t + li][KS * s + KPL * lk];
-            acc[t] = M::run(av, bv, acc[t]);
+#pragma unroll
+            for (int q = 0; q < PW; q++) acc[q][t] = M::run(av, bv[q], acc[q][t]);
           }
         }
       }
@@ -137,7 +149,9 @@ orbital_gemm_kernel(const TI *__restrict__ Ct, int ldc, int n_orb, const TI *__r
     if (ch + 1 < nch) {
       lstore(buf ^ 1);
 #pragma unroll
-      for (int s = 0; s < KC / 4; s++) b[s] = bn[s];
+      for (int q = 0; q < PW; q++)
+#pragma unroll
+        for (int s = 0; s < KC / 4; s++) b[q][s] = bn[q][s];
     }
     __syncthreads();
   }
@@ -147,46 +161,50 @@ orbital_gemm_kernel(const TI *__restrict__ Ct, int ldc, int n_orb, const TI *__r
     // 16x16 tile through LDS so a point's 16 orbitals go out as one segment
     __shared__ TO tile[WPB][16][17];
 #pragma unroll
-    for (int t = 0; t < MT; t++) {
+    for (int qt = 0; qt < PW * MT; qt++) {
+      const int q = qt / MT, t = qt % MT;
 #pragma unroll
-      for (int i = 0; i < 4; i++) tile[wave][li][M::row(lk, i)] = (TO)acc[t][i];
+      for (int i = 0; i < 4; i++) tile[wave][li][M::row(lk, i)] = (TO)acc[q][t][i];
       __syncthreads();
       const int pp = lane >> 2, oo = (lane & 3) * 4;
-      const long p = p0 + pp;
+      const long p = p0 + 16 * q + pp;
       if (live && p < P) {
         TO *dst = out + p * o.s_walker + (long)comp * o.s_comp + o0 + 16 * t + oo;
 #pragma unroll
-        for (int q = 0; q < 4; q++)
-          if (o0 + 16 * t + oo + q < n_orb) dst[q] = tile[wave][pp][oo + q];
+        for (int u = 0; u < 4; u++)
+          if (o0 + 16 * t + oo + u < n_orb) dst[u] = tile[wave][pp][oo + u];
       }
       __syncthreads();
     }
     return;
   }
-  const long p = p0 + li;
-  if (!live || p >= P) return;
-  const long row = p / o.per_walker;
-  const long wk = o.walker_map ? o.walker_map[row] : row;
-  const long pe = (p % o.per_walker) * o.s_elec;
-  if (o.out_val && comp == 0) {
-    double *ov = o.out_val + wk * o.s_walker_val + (p % o.per_walker) * o.s_elec_val;
 #pragma unroll
-    for (int t = 0; t < MT; t++)
+  for (int q = 0; q < PW; q++) {
+    const long p = p0 + 16 * q + li;
+    if (!live || p >= P) return;
+    const long row = p / o.per_walker;
+    const long wk = o.walker_map ? o.walker_map[row] : row;
+    const long pe = (p % o.per_walker) * o.s_elec;
+    if (o.out_val && comp == 0) {
+      double *ov = o.out_val + wk * o.s_walker_val + (p % o.per_walker) * o.s_elec_val;
+#pragma unroll
+      for (int t = 0; t < MT; t++)
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+          const int orb = o0 + 16 * t + M::row(lk, i);
+          if (orb < n_orb) ov[(long)orb * o.s_orb_val] = (double)acc[q][t][i];
+        }
+      continue;
+    }
+    const int oc = o.out_val ? comp - 1 : comp;
+    const long base = (long)oc * o.s_comp + wk * o.s_walker + pe;
+#pragma unroll
+    for (int t = 0; t < MT; t++) {
 #pragma unroll
       for (int i = 0; i < 4; i++) {
         const int orb = o0 + 16 * t + M::row(lk, i);
-        if (orb < n_orb) ov[(long)orb * o.s_orb_val] = (double)acc[t][i];
+        if (orb < n_orb) out[base + (long)orb * o.s_orb] = (TO)acc[q][t][i];
       }
-    return;
-  }
-  const int oc = o.out_val ? comp - 1 : comp;
-  const long base = (long)oc * o.s_comp + wk * o.s_walker + pe;
-#pragma unroll
-  for (int t = 0; t < MT; t++) {
-#pragma unroll
-    for (int i = 0; i < 4; i++) {
-      const int orb = o0 + 16 * t + M::row(lk, i);
-      if (orb < n_orb) out[base + (long)orb * o.s_orb] = (TO)acc[t][i];
     }
   }
 }
@@ -215,28 +233,32 @@ bool gemm_orbital_tiles_valid(int mt, int n_orb, int ldc) {
   return (long)((n_orb + ow - 1) / ow) * ow <= ldc;  // every tile inside the padded orbitals
 }
 
+// Points of a wave.  The coefficients a wave reads from LDS, one read an MFMA,
+// serve all its point tiles: two beyond kSplitRows, where the launch still has
+// several workgroups a CU (17500 rows x 25 orbitals x 266 functions FP64 53.7 ->
+// 50.8 us, and 47.6 with a tile's components on one XCD; 131072 x 128 x 1200
+// FP32 with both 4.4 -> 4.1 ms for the two spins); smaller launches would
+// leave CUs idle.
+template <typename TI, typename TO, int MT, int WPB, int PW>
+static void gemm_launch(const TI *Ct, int ldc, int n_orb, const TI *X, int ldk, long ldp, long P,
+                        int kpad, const GemmOut &o, hipStream_t st) {
+  const unsigned gx = (unsigned)((P + 16 * PW * WPB - 1) / (16 * PW * WPB));
+  hipLaunchKernelGGL((orbital_gemm_kernel<TI, TO, MT, WPB, PW>),
+                     dim3((gx + 7) / 8 * 8 * kComp, (unsigned)((n_orb + 16 * MT - 1) / (16 * MT))),
+                     dim3(64 * WPB), 0, st, Ct, ldc, n_orb, X, ldk, ldp, P, kpad, o);
+}
 template <typename TI, typename TO, int WPB>
 static void gemm_grid(const TI *Ct, int ldc, int n_orb, const TI *X, int ldk, long ldp, long P,
                       int kpad, const GemmOut &o, hipStream_t st, int mt) {
-  const unsigned gx = (unsigned)((P + 16 * WPB - 1) / (16 * WPB));
-  const dim3 blk(64 * WPB);
-  if (mt == 8) {
-    hipLaunchKernelGGL((orbital_gemm_kernel<TI, TO, 8, WPB>),
-                       dim3(gx, kComp, (unsigned)((n_orb + 127) / 128)), blk, 0, st, Ct, ldc,
-                       n_orb, X, ldk, ldp, P, kpad, o);
-  } else if (mt == 4) {
-    hipLaunchKernelGGL((orbital_gemm_kernel<TI, TO, 4, WPB>),
-                       dim3(gx, kComp, (unsigned)((n_orb + 63) / 64)), blk, 0, st, Ct, ldc, n_orb,
-                       X, ldk, ldp, P, kpad, o);
-  } else if (mt == 2) {
-    hipLaunchKernelGGL((orbital_gemm_kernel<TI, TO, 2, WPB>),
-                       dim3(gx, kComp, (unsigned)((n_orb + 31) / 32)), blk, 0, st, Ct, ldc, n_orb,
-                       X, ldk, ldp, P, kpad, o);
-  } else {
-    hipLaunchKernelGGL((orbital_gemm_kernel<TI, TO, 1, WPB>),
-                       dim3(gx, kComp, (unsigned)((n_orb + 15) / 16)), blk, 0, st, Ct, ldc, n_orb,
-                       X, ldk, ldp, P, kpad, o);
-  }
+  const bool wide = WPB == 4 && P > kSplitRows;
+#define QMCB_GEMM(MT)                                                                        \
+  wide ? gemm_launch<TI, TO, MT, WPB, WPB == 4 ? 2 : 1>(Ct, ldc, n_orb, X, ldk, ldp, P, kpad, o, st) \
+       : gemm_launch<TI, TO, MT, WPB, 1>(Ct, ldc, n_orb, X, ldk, ldp, P, kpad, o, st)
+  if (mt == 8) QMCB_GEMM(8);
+  else if (mt == 4) QMCB_GEMM(4);
+  else if (mt == 2) QMCB_GEMM(2);
+  else QMCB_GEMM(1);
+#undef QMCB_GEMM
 }
 
 // wpb: waves (16-point tiles) per workgroup, 4 or 2; mt: 16-orbital tiles
