@@ -188,7 +188,7 @@ hipError_t launch_jastrow_all(const JastrowArgs &a, bool pade_one, const int *wa
 }
 
 // In place of two trace launches, Jastrow, assembly, decision and proposal: 700
-// walkers of 50 electrons 76 -> 40 us a step, 60 of 2 electrons 31 -> 15, an
+// walkers of 50 electrons 76 -> 40 us a step, 128 of 2 electrons 31 -> 15, an
 // evaluate of 1024 x 256 electrons 587 -> 390, of which the traces' inverse and
 // derivatives are 180 at the copy rate.
 //

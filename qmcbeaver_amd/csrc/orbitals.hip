@@ -19,7 +19,7 @@
 // components (its coefficients come straight from L2, one chunk ahead).  The
 // records the stages read come through LDS, loaded two chunks ahead.  The two
 // spins of an all-electron evaluate share a launch where both fit (blockIdx.z):
-// 60 walkers of 2 electrons 15 -> 7.5 us.
+// 128 walkers of 2 electrons 15 -> 7.5 us.
 //
 // Measured, FP32 operands: 1500 points x 75 orbitals x 804 functions 45 us
 // (basis 27 + contraction 39 before), 512 x 100 x 1019 59 us (35 + 52).  A
