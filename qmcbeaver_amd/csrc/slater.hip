@@ -34,7 +34,7 @@ __device__ __forceinline__ void wave_lds_sync() {
 // column to all groups by a lane permute, the largest by DPP, the pivot row
 // through LDS, its reciprocal -- so it is the latency of a step that counts,
 // and many matrices in flight: 700 matrices of 25, both spins' together,
-// 37 us where a workgroup a matrix with two barriers a step took 40 us a
+// 33 us where a workgroup a matrix with two barriers a step took 40 us a
 // spin.  No row is moved: rows are pivoted where they are, and the permutation
 // is undone when the result is written.  ln|det| and sign are accumulated from
 // the pivots and the permutation; the LU of the reference (Crout, implicit
@@ -97,13 +97,6 @@ lu_wave_kernel(SlaterArgs A0, SlaterArgs A1, const int *walkers, int num) {
       if (!(top > 0.0)) {
         sing = true;
       } else {
-        if (r == q) {
-#pragma unroll
-          for (int j = 0; j < C; j++) prow[grp * C + j] = a[j];
-          kr = k;
-        }
-        if (lane == 0) pv[k] = q;
-        wave_lds_sync();
         const double piv = readlane_f64(f, q);
         if (piv < 0) sgn = -sgn;
         if (__builtin_popcount(used >> q) & 1) sgn = -sgn;
@@ -112,14 +105,21 @@ lu_wave_kernel(SlaterArgs A0, SlaterArgs A1, const int *walkers, int num) {
         mant = frexp(mant * fabs(piv), &e2);
         expo += e2;
         const double ip = 1.0 / piv;
-        // the pivot row scaled, the other rows reduced (in place)
+        // the pivot row scaled, the other rows reduced (in place); column k
+        // starts as the unit column, so that the same two operations leave 1/piv
+        // and -f/piv there
+        const bool own = r == q;
+        if (grp == kg) a[kj] = own ? 1.0 : 0.0;
+        if (own) {
 #pragma unroll
-        for (int j = 0; j < C; j++) {
-          const bool own = j == kj && grp == kg;  // column k itself
-          const double pr = own ? ip : prow[grp * C + j] * ip;
-          const double x = own ? -f * ip : __builtin_fma(-f, pr, a[j]);
-          a[j] = r == q ? pr : x;
+          for (int j = 0; j < C; j++) prow[grp * C + j] = a[j] *= ip;
+          kr = k;
         }
+        if (lane == 0) pv[k] = q;
+        wave_lds_sync();
+        const double g = own ? 0.0 : -f;
+#pragma unroll
+        for (int j = 0; j < C; j++) a[j] = __builtin_fma(g, prow[grp * C + j], a[j]);
         wave_lds_sync();
       }
     }
