@@ -21,6 +21,7 @@
 
 #include "qmcb_cusp.hpp"
 #include "qmcb_kernels.hpp"
+#include "qmcb_tiles.hpp"
 
 using namespace qmcb;
 
@@ -249,13 +250,6 @@ uint16_t bf16_bits(float f) {
   if ((u & 0x7fffffffu) > 0x7f800000u) return (uint16_t)((u >> 16) | 0x40u);
   u += 0x7fffu + ((u >> 16) & 1u);
   return (uint16_t)(u >> 16);
-}
-
-int pad_orb(int n) {
-  if (n > 64) return ((n + 127) / 128) * 128;
-  if (n > 32) return 64;
-  if (n > 16) return 32;
-  return 16;
 }
 
 // ---- timing helpers --------------------------------------------------------
