@@ -1144,7 +1144,7 @@ qmcb_status create_impl(const qmcb_system *s, const qmcb_options *o, qmcb_ctx *c
   long cap = std::max<long>(W, std::min<long>(W * std::max(ctx->n[0], 1), (long)(budget / per_point)));
   cap = std::max<long>(cap, std::max(ctx->n[0], 1));
   ctx->ldp = ((cap + 63) / 64) * 64;
-  QCHK(dalloc_bytes(ctx, &ctx->X, per_point * ctx->ldp));
+  QCHK(dalloc_bytes(ctx, &ctx->X, x_elems((long)kComp * ctx->kpad, ctx->ldp) * ctx->tx));
   // device outputs (batch rows)
   qmcb_results &r = ctx->dout;
   QCHK(dalloc(ctx, &r.log_psi, W));
@@ -1425,7 +1425,7 @@ size_t plan_device_bytes(const qmcb_system *s, const qmcb_options *o) {
                                                    : (size_t)1 << 31;
   long cap = std::max<long>(W, std::min<long>(W * std::max(n[0], 1L), (long)(budget / per_point)));
   cap = std::max<long>(cap, std::max(n[0], 1L));
-  add(per_point * (size_t)(((cap + 63) / 64) * 64), 1);
+  add(x_elems((long)kComp * kpad, (cap + 63) / 64 * 64), tx);
   add(W, 8);                                 // log_psi
   add(W, 1);                                 // sign_psi
   add(W * N * 3, 8);

@@ -9,6 +9,15 @@ constexpr int pad_orb(int n) {
   return n > 64 ? (n + 127) / 128 * 128 : n > 32 ? 64 : n > 16 ? 32 : 16;
 }
 
+// Elements of the basis scratch, `rows` rows (functions times components) of ldp
+// points.  A contraction launch reads whole tiles of up to 32 points; those of
+// a walker group start anywhere in a row, so that the last group's last tile
+// may end past the last row.
+constexpr long kPointTile = 32;
+constexpr unsigned long x_elems(long rows, long ldp) {
+  return (unsigned long)(rows * ldp + kPointTile);
+}
+
 // Columns of walk_kernel's tile, by the alpha electrons.
 constexpr int walk_tile(int n) {
   return n <= 16 ? 16 : n <= 32 ? 32 : n <= 64 ? 64 : n <= 96 ? 96 : 128;

@@ -1,7 +1,8 @@
 """Coefficient columns the device walk's FP64 orbital row reads, on the host:
 for every pair of spin sizes each wave's eight columns lie inside the row of the
 moved spin's padded coefficients, and a wave with orbitals of that spin reads
-its own (the tile is the alpha spin's, the row length the moved spin's)."""
+its own (the tile is the alpha spin's, the row length the moved spin's).  Points the
+contraction reads: a walker group's last tile ends inside the basis scratch."""
 import os
 import subprocess
 
@@ -23,6 +24,14 @@ int main() {
           bad += c < 0 || c % 2 != 0 || c + 8 > ldc;  // inside the row, 16-byte aligned
           bad += own < n && c != own;                 // its own orbitals
         }
+    }
+  const long rows = 5 * 64;
+  const long sizes[] = {1, 64, 8192, 16448, 65536, 100032};
+  for (long W : sizes)
+    for (long G = 1; G <= 8 && G <= W; G++) {
+      const long ldp = (W + 63) / 64 * 64, first = W * (G - 1) / G, cnt = W - first;
+      const long last = (rows - 1) * ldp + first + (cnt + 31) / 32 * 32 - 1;
+      bad += last >= (long)x_elems(rows, ldp);
     }
   printf("%d\n", bad);
   return bad != 0;
