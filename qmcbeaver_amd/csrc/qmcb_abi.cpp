@@ -1017,7 +1017,7 @@ qmcb_status create_impl(const qmcb_system *s, const qmcb_options *o, qmcb_ctx *c
     std::vector<double> ct(cnt, 0.0);
     for (int o2 = 0; o2 < n; o2++)
       for (int b = 0; b < ctx->B; b++) ct[(size_t)b * ctx->npad[sp] + o2] = C[(size_t)o2 * ctx->B + b];
-    QCHK(dalloc_bytes(ctx, &ctx->Ct[sp], cnt * ctx->tx));
+    QCHK(dalloc_bytes(ctx, &ctx->Ct[sp], coef_elems(ctx->kpad, ctx->n[0], n) * ctx->tx));
     if (ctx->tx == 8) {
       QCHK(hipMemcpyAsync(ctx->Ct[sp], ct.data(), cnt * 8, hipMemcpyHostToDevice, ctx->stream));
       QCHK(hipStreamSynchronize(ctx->stream));
@@ -1365,7 +1365,7 @@ size_t plan_device_bytes(const qmcb_system *s, const qmcb_options *o) {
   long npad[2];
   for (int sp = 0; sp < 2; sp++) {
     npad[sp] = pad_orb((int)std::max(nact[sp], 1L));
-    add(kpad * npad[sp], tx);
+    add(coef_elems(kpad, (int)n[0], (int)nact[sp]), tx);
     if (tx == 4) add(walk_kpad((int)kpad, 4) * npad[0], 4);  // the walk's copy
   }
   if (o->replace_cusps)

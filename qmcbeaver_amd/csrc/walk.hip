@@ -748,14 +748,12 @@ walk_kernel(WalkArgs A, const int *walkers, int num) {
       // b = 16 i + ks; a basis value read from LDS serves four orbitals
       typedef double d2v __attribute__((ext_vector_type(2)));
       const int ks = lane >> 2, g2_ = 2 * (4 * wave + (lane & 3)), ldc = A.npad[sp];
-      const int lo = walk_row_cols(wave, 0, NC, ldc), hi = walk_row_cols(wave, 1, NC, ldc);
-      const unsigned at = ks * ldc + 2 * (lane & 3);
       double f[4][kComp];
 #pragma unroll
       for (int j = 0; j < 4; j++)
 #pragma unroll
         for (int k = 0; k < kComp; k++) f[j][k] = 0.0;
-      const double *cp = (const double *)A.Ct[sp];
+      const double *cp = (const double *)A.Ct[sp] + (long)ks * ldc + g2_;
       const double *xp = (const double *)X + ks * kXWords<TX>;
       const int ni = kpad / 16;  // even
       constexpr int UD = 2;  // coefficient rows per stage, two stages in flight
@@ -764,8 +762,8 @@ walk_kernel(WalkArgs A, const int *walkers, int num) {
 #pragma unroll
         for (int u = 0; u < UD; u++) {
           const double *p = cp + 16L * (i0 + u) * ldc;
-          q[u][0] = *(const d2v *)(p + lo + at);
-          q[u][1] = *(const d2v *)(p + hi + at);
+          q[u][0] = *(const d2v *)p;
+          q[u][1] = *(const d2v *)(p + NC / 2);  // to column NC - 1 (coef_elems)
         }
       };
       auto mac = [&](int i0, const d2v (*q)[2]) {
