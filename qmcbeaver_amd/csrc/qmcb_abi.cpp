@@ -89,6 +89,8 @@ struct qmcb_ctx {
   int pade_mn = 0, pade_md = 0;   // most terms of any Pade function
   bool pade_one = true;           // every one has one term in each polynomial
   int np_shell = 0;               // primitives, each shell's counted once
+  double *carry = nullptr;        // [Wc][walk_carry_len] block sums of the FP64 walk
+  int *carried = nullptr;         // [Wc] (SlaterArgs)
   float *Cw[2] = {nullptr, nullptr};  // FP32 coefficients as [kpad / 4][npad][4]
   size_t ts = 8, tx = 8, to = 8;  // bytes: derivative storage, GEMM operand, GEMM output
 
@@ -329,6 +331,7 @@ SlaterArgs slater_args(qmcb_ctx *ctx, int sp) {
   a.dcount = ctx->dcount[sp];
   a.ubuf = ctx->ubuf[sp];
   a.zbuf = ctx->zbuf[sp];
+  a.carried = ctx->carried;
   a.ndet = ctx->ndet;
   a.nact = ctx->nact[sp];
   a.occ = ctx->multi ? ctx->d_occ[sp] : nullptr;
@@ -812,6 +815,35 @@ hipError_t upload(qmcb_ctx *ctx, const T **dst, const T *src, size_t count) {
 // padded function count of the walk's rows: FP32 ones run in three stages of 16
 int walk_kpad(int kpad, size_t tx) { return tx == 4 ? (kpad + 47) / 48 * 48 : kpad; }
 
+// Sizes of the walk's tables: primitives (each shell's once) and the most terms
+// of any Pade function; one: every function has one in each polynomial.
+struct WalkTables {
+  int np = 0, mn = 0, md = 0;
+  bool one = true;
+};
+WalkTables walk_tables(const qmcb_system *s, const Shells &sh) {
+  WalkTables t;
+  for (int np : sh.nprim) t.np += np;
+  auto terms = [&](const qmcb_pade &f) {
+    t.mn = std::max(t.mn, (int)f.n_num);
+    t.md = std::max(t.md, (int)f.n_den);
+    if (f.n_num != 1 || f.n_den != 1) t.one = false;
+  };
+  for (const qmcb_pade *f : {&s->ee_updn, &s->ee_upup, &s->ee_dndn}) terms(*f);
+  for (const qmcb_pade *en : {s->en_up, s->en_dn})  // a plan may come without them
+    for (int i = 0; en && i < s->n_nuc; i++) terms(en[i]);
+  return t;
+}
+
+// Whether a context's single-electron walk runs as walk_kernel (kpad, tx: padded
+// functions, bytes of the GEMM operand).
+bool walk_possible(const qmcb_system *s, const qmcb_options *o, const Shells &sh,
+                   const WalkTables &t, int kpad, size_t tx) {
+  return s->n_det <= 1 && !s->occ_up && !s->occ_dn && o->precision != QMCB_MIXED_BF16 &&
+         walk_fits(s->n_up, s->n_basis, walk_kpad(kpad, tx), s->n_nuc, (int)sh.atom.size(), t.np,
+                   t.mn, t.md, tx);
+}
+
 size_t plan_device_bytes(const qmcb_system *s, const qmcb_options *o);
 
 qmcb_status create_impl(const qmcb_system *s, const qmcb_options *o, qmcb_ctx *ctx) {
@@ -880,7 +912,11 @@ qmcb_status create_impl(const qmcb_system *s, const qmcb_options *o, qmcb_ctx *c
   d.nprim = ctx->nprim;
   Shells sh = make_shells(s);
   ctx->nshell = d.nshell = (int)sh.atom.size();
-  for (int np : sh.nprim) ctx->np_shell += np;
+  const WalkTables wt = walk_tables(s, sh);
+  ctx->np_shell = wt.np;
+  ctx->pade_mn = wt.mn;
+  ctx->pade_md = wt.md;
+  ctx->pade_one = wt.one;
   QCHK(upload(ctx, &d.nuc_xyz, s->nuc_xyz, 3 * (size_t)ctx->nn));
   QCHK(upload(ctx, &d.nuc_z, s->nuc_z, (size_t)ctx->nn));
   QCHK(upload(ctx, &d.sh_atom, sh.atom.data(), sh.atom.size()));
@@ -948,16 +984,6 @@ qmcb_status create_impl(const qmcb_system *s, const qmcb_options *o, qmcb_ctx *c
   QCHK(upload(ctx, &d.en[0], s->en_up, (size_t)ctx->nn));
   QCHK(upload(ctx, &d.en[1], s->en_dn, (size_t)ctx->nn));
   QCHK(upload(ctx, &ctx->d_ee, d.ee, 3));  // for kernels that take no DevSystem
-  auto pade_terms = [&](const qmcb_pade &f) {
-    ctx->pade_mn = std::max(ctx->pade_mn, (int)f.n_num);
-    ctx->pade_md = std::max(ctx->pade_md, (int)f.n_den);
-    if (f.n_num != 1 || f.n_den != 1) ctx->pade_one = false;
-  };
-  for (int i = 0; i < 3; i++) pade_terms(d.ee[i]);
-  for (int i = 0; i < ctx->nn; i++) {
-    pade_terms(s->en_up[i]);
-    pade_terms(s->en_dn[i]);
-  }
   double vnn = 0.0;
   for (int i = 0; i < ctx->nn; i++)
     for (int j = i + 1; j < ctx->nn; j++) {
@@ -1004,9 +1030,7 @@ qmcb_status create_impl(const qmcb_system *s, const qmcb_options *o, qmcb_ctx *c
     QCHK(upload(ctx, (const double **)&ctx->d_ci, s->ci_coef, (size_t)ctx->ndet));
   }
 
-  ctx->walk = !ctx->multi && o->precision != QMCB_MIXED_BF16 &&
-              walk_fits(ctx->n[0], ctx->B, walk_kpad(ctx->kpad, ctx->tx), ctx->nn, ctx->nshell, ctx->np_shell,
-                        ctx->pade_mn, ctx->pade_md, ctx->tx);
+  ctx->walk = walk_possible(s, o, sh, wt, ctx->kpad, ctx->tx);
 
   // ---- transposed, padded MO coefficients (active orbitals) in the operand type
   for (int sp = 0; sp < 2; sp++) {
@@ -1097,6 +1121,10 @@ qmcb_status create_impl(const qmcb_system *s, const qmcb_options *o, qmcb_ctx *c
     QCHK(dalloc(ctx, &ctx->dcount[sp], WD));
     QCHK(dalloc(ctx, &ctx->ubuf[sp], W * kDelay * std::max(n, 1L)));
     QCHK(dalloc(ctx, &ctx->zbuf[sp], W * kDelay * std::max(n, 1L)));
+  }
+  if (ctx->walk && walk_carry_len(ctx->n[0], ctx->tx) > 0) {
+    QCHK(dalloc(ctx, &ctx->carry, W * walk_carry_len(ctx->n[0], ctx->tx)));
+    QCHK(dalloc(ctx, &ctx->carried, W));
   }
   QCHK(dalloc(ctx, &ctx->U, W));
   QCHK(dalloc(ctx, &ctx->Ux, W * N * 3));
@@ -1342,12 +1370,11 @@ size_t plan_device_bytes(const qmcb_system *s, const qmcb_options *o) {
   add(3 * B, 4);
   add(std::max(1L, std::min(32L, nshell / 4)) + 1, 4);
   const long nkc = (B + kOrbChunk - 1) / kOrbChunk;
-  long np_shell = 0;
-  for (int np : sh.nprim) np_shell += np;
+  const WalkTables wt = walk_tables(s, sh);
   add(nshell, sizeof(OrbShell));
   add(nkc * kOrbChunk, sizeof(OrbFn));
   add(nkc, sizeof(int4));
-  add(np_shell, sizeof(OrbPrim));
+  add(wt.np, sizeof(OrbPrim));
   add(s->n_prim, 8);
   add(s->n_prim, 8);
   add(nn, sizeof(qmcb_pade));
@@ -1392,6 +1419,11 @@ size_t plan_device_bytes(const qmcb_system *s, const qmcb_options *o) {
     add(WD, 4);
     add(W * kDelay * std::max(n[sp], 1L), 8);
     add(W * kDelay * std::max(n[sp], 1L), 8);
+  }
+  if (const long len = walk_carry_len((int)n[0], tx);
+      len > 0 && walk_possible(s, o, sh, wt, (int)kpad, tx)) {
+    add(W * len, 8);  // the walk's block sums
+    add(W, 4);
   }
   add(W, 8);
   add(W * N * 3, 8);
@@ -1880,6 +1912,10 @@ static WalkArgs walk_args(qmcb_ctx *ctx, long first, int steps, double tau, int 
   a.walk.old_walker = ctx->opt.old_walker_acceptance;
   a.obs = (double *)ctx->vrow;
   a.obs_stride = num;
+  a.carry = ctx->carry;
+  // branching follows the move of electron 0 in DMC; a copied walker would
+  // need its block copied too
+  a.keep = mode == 2 && (first + steps - 1) % ctx->N == 0 ? 0 : 1;
   return a;
 }
 
@@ -2493,6 +2529,7 @@ static CopyArgs walker_copy_args(qmcb_ctx *ctx) {
   add(ctx->cur_el, 8);
   add(ctx->weight, 8);
   add(ctx->age, 4);
+  if (ctx->carried) add(ctx->carried, 4);  // zero after the moves DMC branches at
   if (ctx->ae_drift) {  // the all-electron record
     add(ctx->ae_drift, N * 3 * 8);
     add(ctx->ae_logpsi, 8);

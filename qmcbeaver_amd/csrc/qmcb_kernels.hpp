@@ -140,6 +140,9 @@ struct SlaterArgs {
   //   A^-1 = inv - sum_{a < dcount} ubuf[a] zbuf[a]^T
   int *dcount;           // [Wc]
   double *ubuf, *zbuf;   // [Wc][kDelay][n]
+  // FP64 device walk, or null: nonzero while the walk keeps a walker's block
+  // sums (WalkArgs::carry); whatever else writes an inverse zeroes it
+  int *carried;          // [Wc], both spins'
   // several determinants: the per-determinant arrays above (inv, logdet, sgn,
   // gradPR, lapPR, singular, dcount) are indexed by w * ndet + d, while dval /
   // dmat hold all nact active orbitals of walker w ([Wc][nact][n],
@@ -370,7 +373,14 @@ struct WalkArgs {
   WalkCtl walk;
   double *obs;           // [sweeps of the run][obs_stride][3] observable samples
   long obs_stride;
+  // FP64 operands beyond 32 electrons a spin: T1, T2 and the rows replaced of
+  // the block a run ends in, for the run after it (walk_carry_len doubles a
+  // walker; s[].carried says which walkers have them).  keep 0: dropped.
+  double *carry;
+  int keep;
 };
+// doubles of WalkArgs::carry a walker (0: none are kept)
+long walk_carry_len(int n_up, size_t tx);
 template <typename TS, typename TX>
 hipError_t launch_walk(const WalkArgs &a, const int *walkers, int num, hipStream_t st);
 // whether a system's run fits the kernel's LDS (tx: bytes of the GEMM operand)

@@ -142,6 +142,7 @@ lu_wave_kernel(SlaterArgs A0, SlaterArgs A1, const int *walkers, int num) {
     A.sgn[w] = sing ? 0.0 : sgn;
     A.singular[w] = sing ? 1 : 0;
     A.dcount[w] = 0;
+    if (A.carried) A.carried[w] = 0;
   }
 }
 
@@ -510,6 +511,7 @@ gj_mfma_kernel(SlaterArgs A, const int *walkers, int num) {
     A.sgn[w] = sing ? 0.0 : (pr ? -sg : sg);
     A.singular[w] = sing ? 1 : 0;
     A.dcount[w] = 0;
+    if (A.carried) A.carried[w] = 0;
   }
 }
 
@@ -1378,6 +1380,7 @@ commit_kernel(MoveArgs A, const int *walkers, const uint8_t *mask, int num) {
   for (int i = t; i < 3 * N; i += blockDim.x) Uxw[i] = pUx[i];
   if (t == 0) {
     A.s.dcount[w] = 0;
+    if (A.s.carried) A.s.carried[w] = 0;
     A.s.lapPR[w] = A.st_lap[b];
     A.s.logdet[w] = A.st_logdet[b];
     A.s.sgn[w] = A.st_sgn[b];

@@ -33,6 +33,9 @@
 //     matrices forms T1 and T2 for all of them, and each accepted move updates
 //     both by its rank-one term (T2 of the electrons replaced in the block is
 //     formed from their new rows).  HBM carries the matrices once per KB moves.
+//     A run that ends inside a block leaves its sums in memory and the next one
+//     goes on from them, so that a walk has the same bits however it is cut
+//     into launches (calls, group tuning, other walkers' re-inversions).
 //
 // Steps of a move, seven workgroup barriers: proposal; exponentials (one
 // primitive per thread) and the Jastrow pairs (thread e electron e, and
@@ -414,6 +417,22 @@ walk_kernel(WalkArgs A, const int *walkers, int num) {
       rows = (n + SL - 1) / SL;
       o_beg = sl * rows;
       blk_left = 0;
+      if constexpr (!RD) {
+        const int q = s == 0 ? A.s[sp].carried[w] : 0;
+        if ((q >> 8) == m + 1) {  // go on in the block that the last run ended in
+          const double *cb = A.carry + (long)w * (8 * KB * nu);
+          const int n4 = 4 * n;
+          blk_left = q & 15;
+          nacc = (q >> 4) & 15;
+          if (t < n4) {
+            t1 = cb[t];
+            myacc = (int)cb[n4 + t];
+            for (int i = 0; i < nacc; i++) s_vrow[i * NT + t] = cb[(2 + i) * n4 + t];
+#pragma unroll
+            for (int j = 0; j < KB - 1; j++) G[j] = cb[(1 + KB + j) * n4 + t];
+          }
+        }
+      }
       __syncthreads();
       for (int i = t; i < NC; i += NT)
         if (i >= n)
@@ -1163,6 +1182,21 @@ walk_kernel(WalkArgs A, const int *walkers, int num) {
   }
   // ---- state out
   store_inv(cur);
+  if constexpr (!RD) {
+    const int left = A.keep ? blk_left : 0, n4 = 4 * n;
+    if (left > 0) {
+      double *cb = A.carry + (long)w * (8 * KB * nu);
+      __syncthreads();  // the last move's row in s_vrow
+      if (t < n4) {
+        cb[t] = t1;
+        cb[n4 + t] = myacc;
+        for (int i = 0; i < nacc; i++) cb[(2 + i) * n4 + t] = s_vrow[i * NT + t];
+#pragma unroll
+        for (int j = 0; j < KB - 1; j++) cb[(1 + KB + j) * n4 + t] = G[j];
+      }
+    }
+    if (t == 0) A.s[cur].carried[w] = left > 0 ? left | nacc << 4 | (m_next + 1) << 8 : 0;
+  }
   if (t < N) {
     const long e = (long)w * N + t;
     double *gp = A.s[esp].gradPR + ((long)w * (esp ? N - nu : nu) + ee_) * 3;
@@ -1223,6 +1257,10 @@ bool walk_fits(int n_up, int B, int kpad, int nn, int nshell, int np, int mn, in
   return walk_lds(NC, B, kpad, nn, nshell, np, mn, md, tx) + walk_static_lds(NC) <= kLdsBytes;
 }
 
+long walk_carry_len(int n_up, size_t tx) {
+  return tx == 8 && n_up > 32 ? 8L * walk_block(walk_tile(n_up)) * n_up : 0;
+}
+
 template <typename TS, typename TX, int NC>
 static hipError_t launch_tile(const WalkArgs &a, const int *walkers, int num, hipStream_t st) {
   const size_t lds = walk_lds(NC, a.sys.B, a.kpad, a.sys.nn, a.sys.nshell, a.np, a.pade_mn,
@@ -1242,7 +1280,7 @@ hipError_t launch_walk(const WalkArgs &a, const int *walkers, int num, hipStream
   if (num <= 0 || a.nsteps <= 0) return hipSuccess;
   if (!walk_fits(a.n_up, a.sys.B, a.kpad, a.sys.nn, a.sys.nshell, a.np, a.pade_mn, a.pade_md,
                  sizeof(TX)) ||
-      a.N > 2 * a.n_up)
+      a.N > 2 * a.n_up || (walk_carry_len(a.n_up, sizeof(TX)) > 0 && (!a.carry || !a.s[0].carried)))
     return hipErrorInvalidValue;
   const int NC = walk_tile(a.n_up);
   if (NC == 16) return launch_tile<TS, TX, 16>(a, walkers, num, st);
