@@ -1819,7 +1819,7 @@ struct GroupView {
   hipStream_t stream;
   double *propR, *gauss, *unif, *pU, *pUx, *pUxx, *pVee, *pVen, *d_obs;
   void *X, *vrow;
-  GroupView(qmcb_ctx *c, int g, long first, int sp) : ctx(c) {
+  GroupView(qmcb_ctx *c, int g, long first) : ctx(c) {
     stream = c->stream;
     propR = c->propR; gauss = c->gauss; unif = c->unif;
     pU = c->pU; pUx = c->pUx; pUxx = c->pUxx; pVee = c->pVee; pVen = c->pVen;
@@ -1829,7 +1829,10 @@ struct GroupView {
     c->pU += first; c->pUx += first * c->N * 3; c->pUxx += first; c->pVee += first;
     c->pVen += first; c->d_obs += 3 * first;
     c->X = (char *)c->X + first * c->tx;                                  // point columns
-    c->vrow = (char *)c->vrow + first * (long)kComp * c->npad[sp] * c->to;  // [row][5][npad]
+    // [row][5][npad of the moved spin]: a group's rows where those of the wider
+    // spin would begin, since one group may still read a move's rows while
+    // another writes those of the other spin's first move
+    c->vrow = (char *)c->vrow + first * (long)kComp * std::max(c->npad[0], c->npad[1]) * c->to;
   }
   ~GroupView() {
     ctx->stream = stream;
@@ -2262,7 +2265,7 @@ qmcb_status qmcb_vmc_steps(qmcb_ctx *ctx, int32_t num, int64_t first_step, int32
           WalkArgs ag = a;
           ag.obs += 3 * first;
           if (G > 1) {
-            GroupView view(ctx, g, first, sp);
+            GroupView view(ctx, g, first);
             st = DISPATCH(ctx, walk(ctx, ag, ctx->d_iota + first, (int)cnt));
             if (st == QMCB_OK) st = staggered_refresh(ctx, first, first + cnt, sp);
           } else {
@@ -2296,7 +2299,7 @@ qmcb_status qmcb_vmc_steps(qmcb_ctx *ctx, int32_t num, int64_t first_step, int32
         for (int g = 0; g < G; g++) {
           const long first = (long)num * g / G, cnt = (long)num * (g + 1) / G - first;
           const int *d_map = ctx->d_iota + first;
-          GroupView view(ctx, g, first, sp);
+          GroupView view(ctx, g, first);
           // stagger: group g's front half (proposal, Jastrow, basis, GEMM) of a
           // step starts after group g-1's front half of the same step, so each
           // group trails the one before it and its front overlaps that group's
@@ -2761,7 +2764,7 @@ qmcb_status qmcb_dmc_steps(qmcb_ctx *ctx, int64_t first_step, int32_t n_steps,
     } else if (Geff > 1) {
       for (int g = 0; g < G; g++) {
         const long first = (long)pop * g / G, cnt = (long)pop * (g + 1) / G - first;
-        GroupView view(ctx, g, first, sp);
+        GroupView view(ctx, g, first);
         if (g > 0 && !runs) QCHK(hipStreamWaitEvent(ctx->stream, ctx->gfront[g - 1], 0));
         sst = group_step(first, (int)cnt, g);
         if (sst != QMCB_OK) return sst;
