@@ -203,14 +203,17 @@ int32_t qmcb_abi_version(void);
 
 /* Build a context: copies `sys` to the device and allocates the resident
  * walker state.  Replaces QMCFunctionsFactory::functionsFactory +
- * QMCSCFJastrow::initialize (QMCSCFJastrow.cpp:61-89).  The environment
- * variable QMCB_GEMM_TILE="wpb,mt" (wpb 2 or 4 waves per workgroup, mt 1, 2,
- * 4 or 8 orbital tiles of 16 per wave), read here, makes every batch use the
- * separate basis and orbital GEMM kernels (small ones take a kernel that does
- * both) and fixes the single-electron GEMM's tile instead of the timing
- * autotuner; every choice gives the same bits.  QMCB_SEPARATE_PROPOSE=1 makes the device VMC launch its
- * proposal kernel every step instead of drawing the next proposal inside the
- * move kernel (same bits). */
+ * QMCSCFJastrow::initialize (QMCSCFJastrow.cpp:61-89).  Two environment
+ * variables, read here, choose among kernels.  QMCB_GEMM_TILE="wpb,mt" (wpb 2
+ * or 4 waves per workgroup, mt 1, 2, 4 or 8 orbital tiles of 16 per wave) makes
+ * every batch use the separate basis and orbital GEMM kernels (small ones take
+ * a kernel that does both) and fixes the single-electron GEMM's tile instead of
+ * the timing autotuner; every tile gives the same bits.
+ * QMCB_SEPARATE_PROPOSE=1 makes the device VMC launch its proposal kernel every
+ * step, 0 draws the next proposal inside the move kernel (same bits).  With
+ * either variable set the device walk runs step by step; without, one kernel
+ * carries the walkers of most systems of one determinant through a run of
+ * steps: with FP32 operands the same bits, with FP64 ones equal to rounding. */
 qmcb_status qmcb_create(const qmcb_system *sys, const qmcb_options *opt,
                         qmcb_ctx **out);
 

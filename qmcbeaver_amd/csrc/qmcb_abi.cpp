@@ -83,7 +83,7 @@ struct qmcb_ctx {
   // pair set by QMCB_GEMM_TILE="wpb,mt" at creation ({0, 0}: tuned)
   std::map<std::pair<int, int>, std::pair<int, int>> gemm_tile;
   std::pair<int, int> gemm_force{0, 0};
-  bool separate_propose = false;  // QMCB_SEPARATE_PROPOSE set at creation
+  bool separate_propose = false;  // QMCB_SEPARATE_PROPOSE=1 at creation
   // single-electron walk in one launch per run of steps (walk.hip)
   bool walk = false;
   int pade_mn = 0, pade_md = 0;   // most terms of any Pade function
@@ -836,9 +836,11 @@ WalkTables walk_tables(const qmcb_system *s, const Shells &sh) {
 }
 
 // Whether a context's single-electron walk runs as walk_kernel (kpad, tx: padded
-// functions, bytes of the GEMM operand).
+// functions, bytes of the GEMM operand).  The environment's switches for kernels
+// of the step-by-step walk select that walk.
 bool walk_possible(const qmcb_system *s, const qmcb_options *o, const Shells &sh,
                    const WalkTables &t, int kpad, size_t tx) {
+  if (std::getenv("QMCB_GEMM_TILE") || std::getenv("QMCB_SEPARATE_PROPOSE")) return false;
   return s->n_det <= 1 && !s->occ_up && !s->occ_dn && o->precision != QMCB_MIXED_BF16 &&
          walk_fits(s->n_up, s->n_basis, walk_kpad(kpad, tx), s->n_nuc, (int)sh.atom.size(), t.np,
                    t.mn, t.md, tx);
