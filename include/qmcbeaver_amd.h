@@ -474,7 +474,8 @@ qmcb_status qmcb_property_level(const qmcb_property *p, int32_t level, int64_t *
 
 /* Per-kernel timing of the last qmcb_vmc_steps call, measured with HIP
  * events on the context's stream.  names/ms arrays of length cap; returns
- * the number of entries. */
+ * the number of entries.  "sm_move" counts moves: a launch that carries the
+ * walkers through a run of steps counts as that many. */
 int32_t qmcb_kernel_times(qmcb_ctx *ctx, int32_t cap, const char **names,
                           double *ms, int64_t *launches);
 void qmcb_enable_kernel_timing(qmcb_ctx *ctx, int32_t on);

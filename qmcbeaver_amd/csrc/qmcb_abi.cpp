@@ -31,7 +31,11 @@ namespace {
 thread_local std::string g_create_error;
 
 struct Timing {
-  std::vector<std::pair<int, std::pair<hipEvent_t, hipEvent_t>>> marks;
+  struct Mark {
+    int id, count;  // count: what the timed work counts for (a run of steps: steps)
+    hipEvent_t e0, e1;
+  };
+  std::vector<Mark> marks;
   std::vector<hipEvent_t> pool;
   size_t used = 0;
   std::vector<std::string> names;
@@ -269,7 +273,7 @@ void tm_begin(qmcb_ctx *ctx, const char *name, hipEvent_t *e0) {
   (void)hipEventRecord(*e0, ctx->stream);
   (void)name;
 }
-void tm_end(qmcb_ctx *ctx, const char *name, hipEvent_t e0) {
+void tm_end(qmcb_ctx *ctx, const char *name, hipEvent_t e0, int count) {
   if (!ctx->timing) return;
   Timing &t = ctx->tm;
   hipEvent_t e1 = t.pool[t.used + 1];
@@ -285,7 +289,7 @@ void tm_end(qmcb_ctx *ctx, const char *name, hipEvent_t e0) {
   } else {
     id = it->second;
   }
-  t.marks.push_back({id, {e0, e1}});
+  t.marks.push_back({id, count, e0, e1});
   t.used += 2;
 }
 void tm_collect(qmcb_ctx *ctx) {
@@ -294,20 +298,21 @@ void tm_collect(qmcb_ctx *ctx) {
   (void)hipStreamSynchronize(ctx->stream);
   for (auto &m : t.marks) {
     float ms = 0.f;
-    (void)hipEventElapsedTime(&ms, m.second.first, m.second.second);
-    t.ms[m.first] += ms;
-    t.launches[m.first] += 1;
+    (void)hipEventElapsedTime(&ms, m.e0, m.e1);
+    t.ms[m.id] += ms;
+    t.launches[m.id] += m.count;
   }
   t.marks.clear();
   t.used = 0;
 }
 
-#define TIMED(name, call)               \
+#define TIMED(name, call) TIMED_AS(name, 1, call)
+#define TIMED_AS(name, count, call)     \
   do {                                  \
     hipEvent_t _e0 = nullptr;           \
     tm_begin(ctx, name, &_e0);          \
     hipError_t _r = (call);             \
-    tm_end(ctx, name, _e0);             \
+    tm_end(ctx, name, _e0, count);      \
     if (_r != hipSuccess) {             \
       ctx->err = std::string(name) + ": " + hipGetErrorString(_r); \
       return QMCB_DEVICE_ERROR;         \
@@ -682,10 +687,10 @@ struct Engine {
     return QMCB_OK;
   }
 
-  // a run of single-electron steps in one launch
+  // a run of single-electron steps in one launch, timed as the moves it makes
   static qmcb_status walk(qmcb_ctx *ctx, const WalkArgs &a, const int *d_map, int num) {
     if constexpr (sizeof(TX) >= 4)
-      TIMED("sm_move", (launch_walk<TS, TX>(a, d_map, num, ctx->stream)));
+      TIMED_AS("sm_move", a.nsteps, (launch_walk<TS, TX>(a, d_map, num, ctx->stream)));
     return QMCB_OK;
   }
 
@@ -1932,9 +1937,8 @@ static int walk_sweeps(const qmcb_ctx *ctx, int num) {
 
 // Steps of the run from step `first`, at most `left`: up to the first step
 // after which a re-inversion falls (staggered_refresh), as many sweeps as
-// walk_sweeps allows, one step with kernel timing (per-step launches).
+// walk_sweeps allows.
 static int walk_run_length(const qmcb_ctx *ctx, long first, long left, int num) {
-  if (ctx->timing) return 1;
   const int sweeps = walk_sweeps(ctx, num), K = ctx->rplan_K, S = ctx->rplan_S;
   long mos[2] = {ctx->moves_of_spin[0], ctx->moves_of_spin[1]};
   int rows = 0;

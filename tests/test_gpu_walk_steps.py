@@ -156,3 +156,18 @@ def test_dmc_with_cusps_agrees_with_the_steps(monkeypatch):
     np.testing.assert_array_equal(out[0][0], out[1][0])
     np.testing.assert_allclose(out[1][1], out[0][1], rtol=1e-8, atol=0)
     np.testing.assert_allclose(out[1][2], out[0][2], rtol=0, atol=1e-9 * np.abs(R0).max())
+
+
+def test_kernel_timing_leaves_runs_whole():
+    """With kernel timing a run of steps is still one launch, counted as its
+    steps: one reduction of the samples a call, not one a sweep."""
+    s = synth.make_system(0)
+    W, steps = 64, 40
+    R0, ids = synth.initial_walkers(s, W, 4), np.arange(W)
+    print("case walk timing", flush=True)
+    with Context(s.pack(), precision="fp64", max_walkers=W, seed=2) as c:
+        c.evaluate(ids, R0)
+        k = launches(c, lambda: c.vmc_steps(W, 0, steps, 0.1))
+        rows = c.sample_series()
+    assert k["sm_move"] == steps and k["series"] == 1
+    assert len(rows) == steps // 2
