@@ -1961,10 +1961,10 @@ static int walk_run_length(const qmcb_ctx *ctx, long first, long left, int num) 
 // FP32 operands and 33 to 64 electrons a spin: a workgroup takes a CU, so 256
 // walkers run at once, about 16 us a step, while step by step a batch's time
 // grows less than its size (120 electrons, us a step: 75 against 101 at 1000
-// walkers, 312 against 237 at 4000).  With FP32 operands both ways take a
-// walker through the same bits, so its path does not depend on the choice;
-// with FP64 operands they differ by rounding, and the choice is the system's
-// alone.
+// walkers, 312 against 237 at 4000).  With FP32 operands both ways form a
+// walker's proposals, matrices and gradients with the same bits; the energies
+// and probabilities, whose sums are in another order, agree to rounding.  With
+// FP64 operands everything does, and the choice is the system's alone.
 constexpr int kWalkRounds64 = 4 * 256;
 static bool walk_runs(const qmcb_ctx *ctx, int num) {
   return ctx->walk && (ctx->tx == 8 || ctx->n[0] <= 32 || num <= kWalkRounds64);

@@ -130,9 +130,8 @@ struct WalkCtl {
   double branch_threshold;
 };
 
-// growth: dW^(age+1)
 __device__ inline double reweight_walker(double wt, double dW, int age, double el,
-                                         const WalkCtl &c, double growth) {
+                                         const WalkCtl &c) {
   wt = (c.old_walker > 0 && age - c.old_walker > 0) ? wt * 0.9 : wt * dW;
   const bool bad_energy = c.rel_cutoff > 0.0 && fabs((el - c.e_orig) / c.e_orig) > c.rel_cutoff;
   if (c.equilibrating) {
@@ -141,12 +140,9 @@ __device__ inline double reweight_walker(double wt, double dW, int age, double e
       return 0.0;
     return wt;
   }
+  const double growth = pow(dW, age + 1.0);
   if (growth > 15.0 || dW != dW || wt > 50.0 || bad_energy) return 0.0;
   return wt;
-}
-__device__ inline double reweight_walker(double wt, double dW, int age, double el,
-                                         const WalkCtl &c) {
-  return reweight_walker(wt, dW, age, el, c, pow(dW, age + 1.0));
 }
 
 // ---- wavefront reductions (64 lanes) ---------------------------------------

@@ -102,16 +102,6 @@ __device__ __forceinline__ double quad_sum_own(double v0, double v1, double v2, 
   return keep + dpp_f64<0x4E>(send);
 }
 
-// x^k by squaring (the walk's powers have whole exponents up to a few hundred)
-__device__ __forceinline__ double pow_whole(double x, int k) {
-  double y = 1.0;
-  for (; k > 0; k >>= 1) {
-    if (k & 1) y *= x;
-    x *= x;
-  }
-  return y;
-}
-
 // stored derivatives as the register copy holds them
 template <typename TS> struct DerReg { typedef float T; };
 template <> struct DerReg<double> { typedef double T; };
@@ -1059,8 +1049,7 @@ walk_kernel(WalkArgs A, const int *walkers, int num) {
     double p = sing ? 0.0
                     : exp(2.0 * (logpsi_new - logpsi_old) - (rsum(2) - rsum(1)) / (2.0 * tau));
     if (!(p == p)) p = 0.0;
-    else if (!sing && A.walk.old_walker > 0 && age > A.walk.old_walker)
-      p = age - A.walk.old_walker > 500 ? 1.0 : p * pow_whole(1.1, age - A.walk.old_walker);
+    else if (!sing) p = old_walker_boost(p, age, A.walk.old_walker);
     if (A.mode == 2 && ratio < 0) p = 0.0;
     if (p > 1.0) p = 1.0;
     const bool accept = p > draw[3];
@@ -1091,7 +1080,7 @@ walk_kernel(WalkArgs A, const int *walkers, int num) {
           }
           if (!(p > 0.0)) st_ = 0.0;
           const double dW = exp(A.tau_eff * (p * 0.5 * (so_ + st_) + (1.0 - p) * so_));
-          wt = reweight_walker(wt, dW, age, el, A.walk, pow_whole(dW, age + 1));
+          wt = reweight_walker(wt, dW, age, el, A.walk);
           s_sc[11] = wt;
         }
         s_sc[16] += wt;

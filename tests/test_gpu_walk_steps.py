@@ -171,3 +171,36 @@ def test_kernel_timing_leaves_runs_whole():
         rows = c.sample_series()
     assert k["sm_move"] == steps and k["series"] == 1
     assert len(rows) == steps // 2
+
+
+@pytest.mark.parametrize("n_elec", [38, 76])
+def test_old_walkers_and_weights_either_way(n_elec, monkeypatch):
+    """FP32 operands: walk_kernel and the steps take walkers through the same
+    bits also where ages boost acceptances and decide deletions
+    (old_walker_acceptance 2); weights and samples, whose energies are summed in
+    another order, agree to 1e-12, ln of the ratio of two such sums."""
+    s = synth.make_system(-1, seed=5, n_elec=n_elec)
+    W = 300
+    R0, ids = synth.initial_walkers(s, W, 4), np.arange(W)
+    print("case old walkers", n_elec, flush=True)
+    out = []
+    for env in (None, "0"):
+        with monkeypatch.context() as m:
+            if env:
+                m.setenv("QMCB_SEPARATE_PROPOSE", env)
+            with Context(s.pack(), precision="fp32", max_walkers=2 * W, seed=2, drift_mod=1,
+                         old_walker_acceptance=2) as c:
+                c.evaluate(ids, R0)
+                c.vmc_steps(W, 0, 4 * n_elec + 1, 0.2)
+                rows, R = c.sample_series().copy(), c.positions(W)
+                e = c.evaluate(ids, R)["e_local"]
+                c.dmc_init(W)
+                c.dmc_steps(0, 3 * n_elec + 1, 0.003, float(np.median(e)), target=W,
+                            reweight_after=0, energy_modification=True)
+                slots, wts = c.dmc_population()
+                out.append((R, np.asarray(slots), c.positions(2 * W)[slots], rows,
+                            np.asarray(wts), c.sample_series()))
+    for i in range(3):
+        np.testing.assert_array_equal(out[0][i], out[1][i])
+    for i in range(3, 6):
+        np.testing.assert_allclose(out[0][i], out[1][i], rtol=1e-12, atol=0)
