@@ -1937,13 +1937,14 @@ static int walk_sweeps(const qmcb_ctx *ctx, int num) {
 
 // Steps of the run from step `first`, at most `left`: up to the first step
 // after which a re-inversion falls (staggered_refresh), as many sweeps as
-// walk_sweeps allows.
+// walk_sweeps and as many steps as walk_most_steps allow.
 static int walk_run_length(const qmcb_ctx *ctx, long first, long left, int num) {
   const int sweeps = walk_sweeps(ctx, num), K = ctx->rplan_K, S = ctx->rplan_S;
   long mos[2] = {ctx->moves_of_spin[0], ctx->moves_of_spin[1]};
   int rows = 0;
   long n = 0;
-  while (n < left && n < (1 << 20)) {
+  left = std::min<long>(left, walk_most_steps(ctx->n[0], num));
+  while (n < left) {
     const int m = (int)((first + n) % ctx->N), sp = m < ctx->n[0] ? 0 : 1;
     if (m == 0 && rows == sweeps) break;
     rows += m == 0;

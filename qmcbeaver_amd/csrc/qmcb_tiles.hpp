@@ -33,4 +33,15 @@ constexpr unsigned long coef_elems(long kpad, int n_up, int n) {
   return (unsigned long)(kpad * pad_orb(n) + (over > 0 ? over : 0));
 }
 
+// Most steps of one launch of walk_kernel, about a tenth of a second: other
+// contexts' work on the card waits behind a launch.  A step of `walkers` walkers
+// takes roughly 10 us and 16 + n^2 / 128 ns a walker (n electrons a spin; 8192
+// walkers of 60 electrons, FP32 operands: 152 us, 196 by this; 3000 of 256,
+// FP64: 390 and 442).  A cut costs the state's trip to memory and back, 0.2 ms
+// for the latter.
+constexpr int walk_most_steps(int n, long walkers) {
+  const double us = 10.0 + 1e-3 * walkers * (16.0 + n * n / 128.0);
+  return us < 1e5 ? (int)(1e5 / us) : 1;
+}
+
 }  // namespace qmcb

@@ -1,7 +1,13 @@
-"""Ranges of device reads, on the host.  The device walk's FP64 orbital row loads
-every column of the alpha spin's tile from the moved spin's coefficients: for
-every pair of spin sizes its last element lies inside the array.  Points the
-contraction reads: a walker group's last tile ends inside the basis scratch."""
+"""Ranges of device reads and the length of a walk launch, on the host.
+
+* The device walk's FP64 orbital row loads every column of the alpha spin's tile
+  from the moved spin's coefficients: for every pair of spin sizes its last
+  element lies inside the array.
+* The contraction reads whole tiles of points: a walker group's last one ends
+  inside the basis scratch.
+* A launch of the walk is at least a step and, unless one step is longer, at most
+  a tenth of a second by its own estimate.
+"""
 import os
 import subprocess
 
@@ -27,6 +33,11 @@ int main() {
       const long ldp = (W + 63) / 64 * 64, first = W * (G - 1) / G, cnt = W - first;
       const long last = (rows - 1) * ldp + first + (cnt + 31) / 32 * 32 - 1;
       bad += last >= (long)x_elems(rows, ldp);
+    }
+  for (int n = 1; n <= 128; n++)
+    for (long W = 1; W <= 1000000; W *= 10) {
+      const long steps = walk_most_steps(n, W);
+      bad += steps < 1 || (steps > 1 && steps * (10.0 + W * (16.0 + n * n / 128) / 1e3) > 1e5);
     }
   printf("%d\n", bad);
   return bad != 0;
