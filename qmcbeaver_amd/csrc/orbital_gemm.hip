@@ -233,12 +233,33 @@ bool gemm_orbital_tiles_valid(int mt, int n_orb, int ldc) {
   return (long)((n_orb + ow - 1) / ow) * ow <= ldc;  // every tile inside the padded orbitals
 }
 
-// Points of a wave.  The coefficients a wave reads from LDS, one read an MFMA,
-// serve all its point tiles: two beyond kSplitRows, where the launch still has
-// several workgroups a CU (17500 rows x 25 orbitals x 266 functions FP64 53.7 ->
-// 50.8 us, and 47.6 with a tile's components on one XCD; 131072 x 128 x 1200
-// FP32 with both 4.4 -> 4.1 ms for the two spins); smaller launches would
-// leave CUs idle.
+// Whether a wave takes two point tiles, so that a coefficient it reads from LDS
+// serves both, or one.  Two need up to twice the accumulators: with FP64 operands
+// and more than 32 orbitals one wave is left on a SIMD, which costs more than the
+// reads.  Below, rows x orbitals x functions: us with two and with one.
+//   BF16, up to 64 orbitals: two (66048 x 64 x 670 167 / 182, 20032 39 / 49).
+//   BF16 beyond: one up to 49152 rows (17024 x 128 x 1320 134 / 123, 33024 241 /
+//     236, 66048 484 / 497, 131072 871 / 914; 75 orbitals 76 / 66, 139 / 131, 290 /
+//     282, 517 / 531).
+//   FP32 beyond 64: two (66048 x 128 x 1320 1173 / 1212, 131072 2273 / 2434).
+//   Otherwise two only while their workgroups are at most three a CU, all
+//     running at once (FP64 17000 x 25 x 258 49 / 53, 20000 70 / 61, 66000 242 /
+//     239; FP32 17024 x 64 x 670 97 / 103, 20032 144 / 123, 66048 388 / 359), and
+//     not with FP64 beyond 32 orbitals (17024 x 64 x 670 195 / 182, 66048 x 128 x
+//     1320 2583 / 2393).
+// None at up to kSplitRows rows, where CUs would idle.
+constexpr long kTwoTileGroups = 3 * 256;
+constexpr long kTwoTileRows16 = 3 << 14;
+template <typename TI>
+constexpr bool two_tiles_at(int mt) { return sizeof(TI) < 8 || mt <= 2; }
+template <typename TI>
+static bool two_tiles(int mt, long P, int n_orb) {
+  if (!two_tiles_at<TI>(mt) || P <= kSplitRows) return false;
+  if (sizeof(TI) == 2) return mt < 8 || P > kTwoTileRows16;
+  if (mt == 8) return true;
+  const long gx = (P + 127) / 128, gy = (n_orb + 16 * mt - 1) / (16 * mt);
+  return (gx + 7) / 8 * 8 * kComp * gy <= kTwoTileGroups;
+}
 template <typename TI, typename TO, int MT, int WPB, int PW>
 static void gemm_launch(const TI *Ct, int ldc, int n_orb, const TI *X, int ldk, long ldp, long P,
                         int kpad, const GemmOut &o, hipStream_t st) {
@@ -250,9 +271,10 @@ static void gemm_launch(const TI *Ct, int ldc, int n_orb, const TI *X, int ldk, 
 template <typename TI, typename TO, int WPB>
 static void gemm_grid(const TI *Ct, int ldc, int n_orb, const TI *X, int ldk, long ldp, long P,
                       int kpad, const GemmOut &o, hipStream_t st, int mt) {
-  const bool wide = WPB == 4 && P > kSplitRows;
-#define QMCB_GEMM(MT)                                                                        \
-  wide ? gemm_launch<TI, TO, MT, WPB, WPB == 4 ? 2 : 1>(Ct, ldc, n_orb, X, ldk, ldp, P, kpad, o, st) \
+  const bool wide = WPB == 4 && two_tiles<TI>(mt, P, n_orb);
+#define QMCB_GEMM(MT)                                                                             \
+  wide ? gemm_launch<TI, TO, MT, WPB, WPB == 4 && two_tiles_at<TI>(MT) ? 2 : 1>(                  \
+             Ct, ldc, n_orb, X, ldk, ldp, P, kpad, o, st)                                         \
        : gemm_launch<TI, TO, MT, WPB, 1>(Ct, ldc, n_orb, X, ldk, ldp, P, kpad, o, st)
   if (mt == 8) QMCB_GEMM(8);
   else if (mt == 4) QMCB_GEMM(4);
