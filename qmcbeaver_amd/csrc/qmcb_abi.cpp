@@ -1749,16 +1749,20 @@ qmcb_status qmcb_get_positions(qmcb_ctx *ctx, int32_t num, double *R) {
 }
 
 // The energy accumulators are four arrays one after another in the arena
-// (acc_stride doubles apart): zeroed by one fill and read by one copy.
+// (acc_stride doubles apart).  Where the slots between the first `num` of each
+// are few they are zeroed by one fill and read by one copy: a fill or copy costs
+// about as much as kAccGap bytes.  A call for few walkers of a context of many
+// takes each array's own part.
 static size_t acc_stride(const qmcb_ctx *ctx) { return arena_round(8 * (size_t)ctx->Wc) / 8; }
-static bool acc_block(const qmcb_ctx *ctx) {
+constexpr size_t kAccGap = (size_t)128 << 10;
+static bool acc_block(const qmcb_ctx *ctx, int num) {
   const size_t s = acc_stride(ctx);
-  return ctx->acc_el2 == ctx->acc_el + s && ctx->acc_n == ctx->acc_el + 2 * s &&
-         ctx->acc_prop_el == ctx->acc_el + 3 * s;
+  return 8 * (s - num) <= kAccGap && ctx->acc_el2 == ctx->acc_el + s &&
+         ctx->acc_n == ctx->acc_el + 2 * s && ctx->acc_prop_el == ctx->acc_el + 3 * s;
 }
 static hipError_t zero_acc(qmcb_ctx *ctx, int num, bool weights) {
   hipError_t e = hipSuccess;
-  if (acc_block(ctx)) {
+  if (acc_block(ctx, num)) {
     e = hipMemsetAsync(ctx->acc_el, 0, 8 * (3 * acc_stride(ctx) + num), ctx->stream);
   } else {
     for (double *p : {ctx->acc_el, ctx->acc_el2, ctx->acc_n, ctx->acc_prop_el})
@@ -1772,14 +1776,15 @@ static hipError_t zero_acc(qmcb_ctx *ctx, int num, bool weights) {
 // stream synchronised
 static hipError_t get_acc(qmcb_ctx *ctx, int num, std::vector<double> &own, const double *&el,
                           const double *&el2, const double *&n, const double *&prop) {
-  const size_t s = acc_stride(ctx), all = 3 * s + num;
+  const bool block = acc_block(ctx, num);
+  const size_t s = block ? acc_stride(ctx) : num, all = 3 * s + num;
   double *h = (double *)pin_reserve(ctx, 8 * all);
   if (!h) {
     own.resize(all);
     h = own.data();
   }
   hipError_t e = hipSuccess;
-  if (acc_block(ctx)) {
+  if (block) {
     e = hipMemcpyAsync(h, ctx->acc_el, 8 * all, hipMemcpyDeviceToHost, ctx->stream);
   } else {
     const double *src[4] = {ctx->acc_el, ctx->acc_el2, ctx->acc_n, ctx->acc_prop_el};
