@@ -154,25 +154,14 @@ class ResultArrays:
 
     def __init__(self, num: int, N: int):
         self.num, self.N = num, N
-        # one block, each array on an 8-byte boundary (the entry point fills
-        # every array it is given)
-        shapes = [(f, np.int8, (num,)) if f in ("sign_psi", "singular")
-                  else (f, np.float64, {"grad_lnpsi": (num, N, 3), "mod_drift": (num, N, 3),
-                                        "r2": (num, 3)}.get(f, (num,)))
-                  for f in self.FIELDS]
-        words = [(int(np.prod(sh)) * np.dtype(dt).itemsize + 7) // 8 for _, dt, sh in shapes]
-        block = np.zeros(sum(words) + 1)
-        base, at = block.ctypes.data, 0
-        self.a, ptrs = {}, np.empty(len(shapes), dtype=np.uint64)
-        for i, ((f, dt, sh), w) in enumerate(zip(shapes, words)):
-            v = block[at:at + w]
-            if dt is np.int8:
-                v = v.view(np.int8)[:num]
-            self.a[f] = v.reshape(sh)
-            ptrs[i] = base + 8 * at
-            at += w
-        self._block = block
-        self.struct = Results.from_buffer_copy(ptrs)
+        # an allocation each, so that a caller who keeps one array keeps no other
+        self.a = {f: np.zeros((num, N, 3) if f in ("grad_lnpsi", "mod_drift") else
+                              (num, 3) if f == "r2" else num,
+                              dtype=np.int8 if f in ("sign_psi", "singular") else np.float64)
+                  for f in self.FIELDS}
+        # Results' pointers in its fields' order
+        self.struct = Results.from_buffer_copy(
+            np.array([v.ctypes.data for v in self.a.values()], dtype=np.uint64))
 
     def row(self, i: int) -> "Results":
         """Results struct addressing row i only (for single-walker oracle calls)."""
