@@ -1066,6 +1066,7 @@ qmcb_status create_impl(const qmcb_system *s, const qmcb_options *o, qmcb_ctx *c
       for (size_t i = 0; i < cnt; i++) cf[i] = (float)ct[i];
       QCHK(hipMemcpyAsync(ctx->Ct[sp], cf.data(), cnt * 4, hipMemcpyHostToDevice, ctx->stream));
       QCHK(hipStreamSynchronize(ctx->stream));
+      if (!ctx->walk) continue;
       // four consecutive functions of an orbital together, for the walk's rows
       // (both spins as wide as the alpha spin's padded orbitals)
       const size_t np = ctx->npad[sp], wide = ctx->npad[0], cnw = (size_t)walk_kpad(ctx->kpad, 4) * wide;
@@ -1378,6 +1379,7 @@ size_t plan_device_bytes(const qmcb_system *s, const qmcb_options *o) {
   add(std::max(1L, std::min(32L, nshell / 4)) + 1, 4);
   const long nkc = (B + kOrbChunk - 1) / kOrbChunk;
   const WalkTables wt = walk_tables(s, sh);
+  const bool walks = walk_possible(s, o, sh, wt, (int)kpad, tx);
   add(nshell, sizeof(OrbShell));
   add(nkc * kOrbChunk, sizeof(OrbFn));
   add(nkc, sizeof(int4));
@@ -1400,7 +1402,7 @@ size_t plan_device_bytes(const qmcb_system *s, const qmcb_options *o) {
   for (int sp = 0; sp < 2; sp++) {
     npad[sp] = pad_orb((int)std::max(nact[sp], 1L));
     add(coef_elems(kpad, (int)n[0], (int)nact[sp]), tx);
-    if (tx == 4) add(walk_kpad((int)kpad, 4) * npad[0], 4);  // the walk's copy
+    if (tx == 4 && walks) add(walk_kpad((int)kpad, 4) * npad[0], 4);  // the walk's copy
   }
   if (o->replace_cusps)
     for (int sp = 0; sp < 2; sp++) {
@@ -1427,8 +1429,7 @@ size_t plan_device_bytes(const qmcb_system *s, const qmcb_options *o) {
     add(W * kDelay * std::max(n[sp], 1L), 8);
     add(W * kDelay * std::max(n[sp], 1L), 8);
   }
-  if (const long len = walk_carry_len((int)n[0], tx);
-      len > 0 && walk_possible(s, o, sh, wt, (int)kpad, tx)) {
+  if (const long len = walk_carry_len((int)n[0], tx); len > 0 && walks) {
     add(W * len, 8);  // the walk's block sums
     add(W, 4);
   }

@@ -161,8 +161,7 @@ __host__ __device__ constexpr int walk_slices() {
   return sizeof(TX) == 8 || NC == 16 ? 4 : 2;
 }
 // groups of threads that share a column's four derivative components (each
-// with the column of A^-1): two where that keeps a thread within 256
-// registers (32 and 64 columns; the wider tiles' columns alone need more)
+// with the column of A^-1), FP32 operands: what keeps a thread near 256 registers
 template <typename TX, int NC>
 __host__ __device__ constexpr int walk_groups() {
   return sizeof(TX) == 8 || NC == 16 ? 1 : (NC == 32 ? 2 : 4);
@@ -174,11 +173,7 @@ __host__ __device__ constexpr int walk_threads() {
 // whether the moved spin's derivative matrices are held in registers
 template <typename TX>
 __host__ __device__ constexpr bool der_in_reg(int NC) { return sizeof(TX) == 4 || NC <= 32; }
-// waves per SIMD the register allocation must allow
-template <typename TS, typename TX, int NC>
-__host__ __device__ constexpr int walk_waves() {
-  return 2;
-}
+constexpr int kWalkWaves = 2;  // waves per SIMD the register allocation must allow
 
 // drift_factor_near with the nucleus {x, y, z, Z} in LDS
 __device__ __forceinline__ double drift_factor_lds(const double g[3], const double x[3],
@@ -206,9 +201,6 @@ __device__ __forceinline__ double wave_min(double v) {
               fmin(readlane_f64(v, 32), readlane_f64(v, 48)));
 }
 
-// orbitals of a row of Cw: the alpha spin's padded count
-__host__ __device__ constexpr int walk_row_width(int NC) { return NC == 96 ? 128 : NC; }
-
 // the quad's values added in lane order, ((0 + 1) + 2) + 3
 __device__ __forceinline__ double quad_ordered(double v) {
   return ((quad_bcast<0>(v) + quad_bcast<1>(v)) + quad_bcast<2>(v)) + quad_bcast<3>(v);
@@ -224,7 +216,7 @@ __device__ __forceinline__ double quad_ordered_own(double v0, double v1, double 
 template <typename TS, typename TX, int NC>
 __global__ void
 __attribute__((amdgpu_flat_work_group_size(walk_threads<TX, NC>(), walk_threads<TX, NC>()),
-               amdgpu_waves_per_eu(walk_waves<TS, TX, NC>())))
+               amdgpu_waves_per_eu(kWalkWaves)))
 walk_kernel(WalkArgs A, const int *walkers, int num) {
   constexpr int NT = walk_threads<TX, NC>(), NW = NT / 64, SL = walk_slices<TX, NC>(), KB = walk_block(NC);
   constexpr int RI = NC / SL;   // most rows of a slice
@@ -646,12 +638,11 @@ walk_kernel(WalkArgs A, const int *walkers, int num) {
     constexpr int UB = 4;  // groups of four functions per stage, three stages in flight
     const int og = 32 * wave;
     f4 cq[F32 ? 3 : 1][F32 ? UB : 1];
-    constexpr int NPW = walk_row_width(NC);
-    const f4 *cw = (const f4 *)A.Cw[sp] + min(og + (lane & 31), NPW - 1);
+    const f4 *cw = (const f4 *)A.Cw[sp] + min(og + (lane & 31), NC - 1);
     auto row_load = [&](int g0, f4 *q) {
-      const f4 *p = cw + g0 * NPW;
+      const f4 *p = cw + g0 * NC;
 #pragma unroll
-      for (int u = 0; u < UB; u++) q[u] = p[u * NPW];
+      for (int u = 0; u < UB; u++) q[u] = p[u * NC];
     };
     // ---- basis functions, one per thread: radial sums, then the product rule
     for (int j = t; j < B; j += NT) {
