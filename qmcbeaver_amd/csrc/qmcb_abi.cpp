@@ -846,6 +846,7 @@ WalkTables walk_tables(const qmcb_system *s, const Shells &sh) {
 bool walk_possible(const qmcb_system *s, const qmcb_options *o, const Shells &sh,
                    const WalkTables &t, int kpad, size_t tx) {
   if (std::getenv("QMCB_GEMM_TILE") || std::getenv("QMCB_SEPARATE_PROPOSE")) return false;
+  if (o->all_electron_moves) return false;  // takes no single-electron steps
   return s->n_det <= 1 && !s->occ_up && !s->occ_dn && o->precision != QMCB_MIXED_BF16 &&
          walk_fits(s->n_up, s->n_basis, walk_kpad(kpad, tx), s->n_nuc, (int)sh.atom.size(), t.np,
                    t.mn, t.md, tx);

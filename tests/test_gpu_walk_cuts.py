@@ -126,3 +126,16 @@ def test_plan_counts_the_kept_sums(precision):
     print("case walk plan", precision, flush=True)
     with Context(p, precision=precision, max_walkers=77) as c:
         assert c.device_bytes() == plan_device_bytes(p, precision=precision, max_walkers=77)
+
+
+def test_all_electron_contexts_hold_no_kept_sums():
+    p = system(50, 40)
+    W, held = 1000, []
+    print("case walk memory, all-electron moves", flush=True)
+    for every in (False, True):
+        with Context(p, precision="fp64", max_walkers=W, all_electron_moves=every) as c:
+            held.append(c.device_bytes())
+            c.evaluate(np.arange(8), walkers(p, 8, 3))
+            assert np.isfinite(c.vmc_steps(8, 0, 3, 0.01).sum_e_local)
+    # a block's sums, 8 x 8 x 50 numbers a walker, against a record of 3 x 90 + 4
+    assert held[1] < held[0]
