@@ -848,7 +848,7 @@ bool walk_possible(const qmcb_system *s, const qmcb_options *o, const Shells &sh
   if (std::getenv("QMCB_GEMM_TILE") || std::getenv("QMCB_SEPARATE_PROPOSE")) return false;
   if (o->all_electron_moves) return false;  // takes no single-electron steps
   return s->n_det <= 1 && !s->occ_up && !s->occ_dn && o->precision != QMCB_MIXED_BF16 &&
-         walk_fits(s->n_up, s->n_basis, walk_kpad(kpad, tx), s->n_nuc, (int)sh.atom.size(), t.np,
+         walk_fits(s->n_up, s->n_dn, s->n_basis, walk_kpad(kpad, tx), s->n_nuc, (int)sh.atom.size(), t.np,
                    t.mn, t.md, tx);
 }
 
@@ -1969,10 +1969,10 @@ static int walk_run_length(const qmcb_ctx *ctx, long first, long left, int num) 
 // FP32 operands and 33 to 64 electrons a spin: a workgroup takes a CU, so 256
 // walkers run at once, about 16 us a step, while step by step a batch's time
 // grows less than its size (120 electrons, us a step: 75 against 101 at 1000
-// walkers, 312 against 237 at 4000).  With FP32 operands both ways form a
-// walker's proposals, matrices and gradients with the same bits; the energies
-// and probabilities, whose sums are in another order, agree to rounding.  With
-// FP64 operands everything does, and the choice is the system's alone.
+// walkers, 312 against 237 at 4000).  There both ways form a walker's
+// proposals, matrices and gradients with the same bits; the energies and
+// probabilities, whose sums are in another order, agree to rounding.  With FP64
+// operands everything does, and the choice is the system's alone.
 constexpr int kWalkRounds64 = 4 * 256;
 static bool walk_runs(const qmcb_ctx *ctx, int num) {
   return ctx->walk && (ctx->tx == 8 || ctx->n[0] <= 32 || num <= kWalkRounds64);

@@ -385,7 +385,7 @@ template <typename TS, typename TX>
 hipError_t launch_walk(const WalkArgs &a, const int *walkers, int num, hipStream_t st);
 // whether a system's run fits the kernel's LDS (tx: bytes of the GEMM operand)
 // (np: primitives, each shell's counted once)
-bool walk_fits(int n_up, int B, int kpad, int nn, int nshell, int np, int mn, int md, size_t tx);
+bool walk_fits(int n_up, int n_dn, int B, int kpad, int nn, int nshell, int np, int mn, int md, size_t tx);
 
 // ---- kernel (d): Jastrow + Coulomb, all-electron and single-electron ----
 struct JastrowArgs {

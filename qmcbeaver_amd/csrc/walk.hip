@@ -155,7 +155,9 @@ __device__ __forceinline__ int x_at(int j) {
 // basis values are rounded to FP32, so a last-bit change of an FP64 sum can
 // flip a rounding and be seen 2^-24 large: every sum that feeds a position or a
 // stored row keeps sm_move_kernel's order (its slices, rows ascending within
-// one, slices added in order).  FP64 operands take four slices throughout.
+// one, slices added in order; the tile being the alpha spin's, up to 16 beta
+// electrons under more alpha ones have other slices than there).  FP64 operands
+// take four slices throughout.
 template <typename TX, int NC>
 __host__ __device__ constexpr int walk_slices() {
   return sizeof(TX) == 8 || NC == 16 ? 4 : 2;
@@ -1224,7 +1226,7 @@ size_t walk_static_lds(int NC) {
 
 }  // namespace
 
-bool walk_fits(int n_up, int B, int kpad, int nn, int nshell, int np, int mn, int md, size_t tx) {
+bool walk_fits(int n_up, int n_dn, int B, int kpad, int nn, int nshell, int np, int mn, int md, size_t tx) {
   if (n_up < 1 || n_up > 128 || (tx != 8 && tx != 4)) return false;
   // FP32 operands beyond 64 electrons a spin: the columns of A^-1 and the
   // derivative matrices, in the two slices the bits ask for, are more than a
@@ -1232,6 +1234,10 @@ bool walk_fits(int n_up, int B, int kpad, int nn, int nshell, int np, int mn, in
   // for 16 steps in two rounds of 256, 2.9 ms step by step; 8192 walkers of
   // 256 electrons: 1.7 against 0.93 ms a step)
   if (tx == 4 && n_up > 64) return false;
+  // Beyond 32 electrons a spin the batch decides between this kernel and the
+  // steps, which then have to give a walker the same bits: they do with the same
+  // slices of a column, two but in the steps' 16-column tile, which has four
+  if (tx == 4 && n_up > 32 && n_dn > 0 && n_dn <= 16) return false;
   if (np >= 1 << 16 || nn >= 1 << 20 || kpad % (tx == 4 ? 48 : 32)) return false;  // packed function records
   const int NC = walk_tile(n_up);
   return walk_lds(NC, B, kpad, nn, nshell, np, mn, md, tx) + walk_static_lds(NC) <= kLdsBytes;
@@ -1258,7 +1264,7 @@ static hipError_t launch_tile(const WalkArgs &a, const int *walkers, int num, hi
 template <typename TS, typename TX>
 hipError_t launch_walk(const WalkArgs &a, const int *walkers, int num, hipStream_t st) {
   if (num <= 0 || a.nsteps <= 0) return hipSuccess;
-  if (!walk_fits(a.n_up, a.sys.B, a.kpad, a.sys.nn, a.sys.nshell, a.np, a.pade_mn, a.pade_md,
+  if (!walk_fits(a.n_up, a.N - a.n_up, a.sys.B, a.kpad, a.sys.nn, a.sys.nshell, a.np, a.pade_mn, a.pade_md,
                  sizeof(TX)) ||
       a.N > 2 * a.n_up || (walk_carry_len(a.n_up, sizeof(TX)) > 0 && (!a.carry || !a.s[0].carried)))
     return hipErrorInvalidValue;

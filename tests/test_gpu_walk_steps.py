@@ -204,3 +204,18 @@ def test_old_walkers_and_weights_either_way(n_elec, monkeypatch):
         np.testing.assert_array_equal(out[0][i], out[1][i])
     for i in range(3, 6):
         np.testing.assert_allclose(out[0][i], out[1][i], rtol=1e-12, atol=0)
+
+
+@pytest.mark.parametrize("n_up,n_dn", [(40, 9), (64, 16), (40, 17), (33, 0)])
+def test_same_bits_either_side_of_the_batch_rule(n_up, n_dn):
+    """FP32 operands, 33 to 64 up electrons: walkers among 1000 and among 1040."""
+    p = system(n_up, n_dn)
+    R0 = walkers(p, 1040, 5)
+    print("case batch rule", n_up, n_dn, flush=True)
+    out = []
+    for W in (1000, 1040):
+        with Context(p, precision="fp32", max_walkers=W, seed=4, drift_mod=1) as c:
+            c.evaluate(np.arange(W), R0[:W])
+            c.vmc_steps(W, n_up - 10, 60, 0.02)
+            out.append(c.positions(W)[:1000])
+    np.testing.assert_array_equal(out[0], out[1])
