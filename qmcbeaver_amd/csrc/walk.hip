@@ -227,6 +227,10 @@ walk_kernel(WalkArgs A, const int *walkers, int num) {
   constexpr int NK = KC >= SL ? KC / SL : 1;  // components a lane of a column sums up
   constexpr bool ONE = KC < SL;               // one component, the same in both lanes
   constexpr bool F32 = sizeof(TX) == 4, RD = der_in_reg<TX>(NC);
+  // stored derivatives narrower than the row they come from: a move's own traces
+  // take the row as formed, every later one as stored, which in a block is T1 and
+  // T2 of the electrons replaced
+  constexpr bool NARROW = !RD && sizeof(TS) < sizeof(TX);
   typedef typename DerReg<TS>::T TD;
   const int b = blockIdx.x;
   if (b >= num) return;
@@ -247,7 +251,7 @@ walk_kernel(WalkArgs A, const int *walkers, int num) {
   __shared__ double s_wj[7][NW], s_red[8][NW];
   __shared__ double s_draw[64][4];     // three normal deviates, one uniform
   __shared__ double s_xn[2][3], s_xo[2][3];
-  __shared__ double s_new[4];
+  __shared__ double s_new[4], s_held[4];  // the moved electron's T1 ratio, NARROW: of its stored row
   __shared__ double s_fix[KB][4];
   __shared__ double s_sc[17];  // thread 0's scalars, below
   __shared__ double s_psi[2][3];  // U and ln|det| of either spin, by step parity
@@ -939,6 +943,20 @@ walk_kernel(WalkArgs A, const int *walkers, int num) {
       if (lane == 0)
 #pragma unroll
         for (int k = 0; k < 4; k++) s_new[k] = f[k];
+      if constexpr (NARROW) {
+#pragma unroll
+        for (int k = 0; k < 4; k++) f[k] = 0.0;
+#pragma unroll
+        for (int h = 0; h < (NC + 63) / 64; h++)
+          if (lane + 64 * h < n)
+#pragma unroll
+            for (int k = 0; k < 4; k++) f[k] += (double)(TS)s_v[1 + k][lane + 64 * h] * col[cl[h]];
+#pragma unroll
+        for (int k = 0; k < 4; k++) f[k] = wave_sum(f[k]);
+        if (lane == 0)
+#pragma unroll
+          for (int k = 0; k < 4; k++) s_held[k] = f[k];
+      }
     }
     __syncthreads();
     const double ratio = s_wv[r];
@@ -1116,7 +1134,7 @@ walk_kernel(WalkArgs A, const int *walkers, int num) {
         }
       }
       if constexpr (!RD) {
-        t1 = gown[0];
+        t1 = NARROW && c == r ? s_held[sl] * qinv : gown[0];
         if (c == r) myacc = nacc;
       }
       fo = ft;
@@ -1136,7 +1154,7 @@ walk_kernel(WalkArgs A, const int *walkers, int num) {
         st_der(dmw + 4 * ((long)o * n + r), v4[0], v4[1], v4[2], v4[3]);
         if constexpr (!RD)
 #pragma unroll
-          for (int k = 0; k < 4; k++) s_vrow[(nacc * NC + o) * 4 + k] = as_stored<TS>(v4[k]);
+          for (int k = 0; k < 4; k++) s_vrow[(nacc * NC + o) * 4 + k] = (double)(TS)v4[k];
       }
       if constexpr (RD) {
         if (c == r) {
@@ -1220,7 +1238,7 @@ size_t walk_lds(int NC, int B, int kpad, int nn, int nshell, int np, int mn, int
 constexpr size_t kLdsBytes = 160 * 1024;
 // the kernel's static LDS, an upper bound over the tiles
 size_t walk_static_lds(int NC) {
-  return 8 * (size_t)(2 * NC + kComp * NC + NC + 4 * NC + 15 * 8 + 64 * 4 + 12 + 4 + 4 * 8 + 23) +
+  return 8 * (size_t)(2 * NC + kComp * NC + NC + 4 * NC + 15 * 8 + 64 * 4 + 12 + 8 + 4 * 8 + 23) +
          256;
 }
 
