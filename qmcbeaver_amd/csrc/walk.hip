@@ -12,8 +12,8 @@
 // walker's whole spin state (A^-1 and four derivative matrices) from HBM.  In
 // one launch a step is a chain of LDS round trips, FP64 divisions, square
 // roots, exponentials and wave sums of about 17 k cycles for two electrons and
-// 30 k for 64, with the moved spin's state on chip from move to move.  Time of
-// a step, before (four launches) and now: 2 electrons x 128 walkers FP64 33.7
+// 32 k for 64 (waits are 35 and 42 % of them, vector instructions 46 and 33), with
+// the moved spin's state on chip from move to move.  Time of a step, before (four launches) and now: 2 electrons x 128 walkers FP64 33.7
 // and 8.8 us; 38 x 61 mixed 50.9 and 12.7; 122 x 50 mixed with cusps (DMC) 102
 // and 25; 64 x 1024 FP64 73 and 16; 256 x 3000 FP64 692 and 390; 60 x 8192
 // mixed 184 and 152.
@@ -31,8 +31,9 @@
 //   FP64 operands beyond: the moves run electron by electron, so the columns
 //     r, r+1, ... of the next KB moves are known: one pass over the derivative
 //     matrices forms T1 and T2 for all of them, and each accepted move updates
-//     both by its rank-one term (T2 of the electrons replaced in the block is
-//     formed from their new rows).  HBM carries the matrices once per KB moves.
+//     both by its rank-one term (T1 and T2 of the electrons replaced in the block
+//     are formed from their new rows as stored).  The matrices are read once per
+//     KB moves.
 //     A run that ends inside a block leaves its sums in memory and the next one
 //     goes on from them, so that a walk has the same bits however it is cut
 //     into launches (calls, group tuning, other walkers' re-inversions).
@@ -49,7 +50,9 @@
 // The random numbers of 64 steps are drawn at once, one step per lane.
 // LDS reads are requested in groups ahead of a scheduling barrier: left to
 // itself the compiler (with the flags that keep this loop's constants out of
-// registers) waits on each one, 130 cycles a read.
+// registers) waits on each one, 130 cycles a read.  The FP32 64-column tile
+// spills 46 to 56 registers in the loop (112 to 120 bytes a lane); no other tile
+// spills vector registers, and every one keeps 75 to 225 scalars in their lanes.
 #include "qmcb_cusp.hpp"
 #include "qmcb_kernels.hpp"
 #include "qmcb_pade.hpp"
@@ -931,32 +934,22 @@ walk_kernel(WalkArgs A, const int *walkers, int num) {
       }
       if (sl == 0 && c < n && grp == 0) s_wv[c] = wc;
     }
-    if (wave == 0) {
+    if (wave == 0 || (NARROW && wave == 1)) {
+      const bool held = NARROW && wave == 1;
       double f[4] = {0, 0, 0, 0};
 #pragma unroll
       for (int h = 0; h < (NC + 63) / 64; h++)
         if (lane + 64 * h < n)
 #pragma unroll
-          for (int k = 0; k < 4; k++) f[k] += as_stored<TS>(s_v[1 + k][lane + 64 * h]) * col[cl[h]];
+          for (int k = 0; k < 4; k++) {
+            const double x = s_v[1 + k][lane + 64 * h];
+            f[k] += (held ? (double)(TS)x : as_stored<TS>(x)) * col[cl[h]];
+          }
 #pragma unroll
       for (int k = 0; k < 4; k++) f[k] = wave_sum(f[k]);
       if (lane == 0)
 #pragma unroll
-        for (int k = 0; k < 4; k++) s_new[k] = f[k];
-      if constexpr (NARROW) {
-#pragma unroll
-        for (int k = 0; k < 4; k++) f[k] = 0.0;
-#pragma unroll
-        for (int h = 0; h < (NC + 63) / 64; h++)
-          if (lane + 64 * h < n)
-#pragma unroll
-            for (int k = 0; k < 4; k++) f[k] += (double)(TS)s_v[1 + k][lane + 64 * h] * col[cl[h]];
-#pragma unroll
-        for (int k = 0; k < 4; k++) f[k] = wave_sum(f[k]);
-        if (lane == 0)
-#pragma unroll
-          for (int k = 0; k < 4; k++) s_held[k] = f[k];
-      }
+        for (int k = 0; k < 4; k++) (held ? s_held : s_new)[k] = f[k];
     }
     __syncthreads();
     const double ratio = s_wv[r];
