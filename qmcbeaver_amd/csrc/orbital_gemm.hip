@@ -59,11 +59,17 @@ orbital_gemm_kernel(const TI *__restrict__ Ct, int ldc, int n_orb, const TI *__r
   __shared__ TI cs[2][LR][LW];
   const int tid = threadIdx.x;
   const int lane = tid & 63, wave = tid >> 6;
-  // the components of a point tile on one XCD, one after another (workgroups go
-  // to the eight XCDs in turn): an element's derivatives, four components, are
-  // one store of the L2 they meet in
-  const int local = blockIdx.x >> 3, comp = local % kComp;
-  const long p0 = (((long)(local / kComp) * 8 + (blockIdx.x & 7)) * WPB + wave) * 16 * PW;
+  // All electrons: the components of a point tile on one XCD, one after another
+  // (workgroups go to the eight XCDs in turn): an element's derivatives, four
+  // components, are one store of the L2 they meet in.  A moved electron's rows,
+  // which do not meet, go component by component (8192 walkers of 256 electrons in
+  // three groups, 256 moves beside sm_move: 239.8 ms, 244.1 the other way).
+  const bool meet = o.out_val != nullptr;
+  const int tiles = gridDim.x / kComp, local = blockIdx.x >> 3;
+  const int comp = meet ? local % kComp : blockIdx.x / tiles;
+  const long tile = meet ? (long)(local / kComp) * 8 + (blockIdx.x & 7) : blockIdx.x % tiles;
+  const long p0 = (tile * WPB + wave) * 16 * PW;
+  if (tile * WPB * 16 * PW >= P) return;  // of the rounding to eight tiles
   const bool live = p0 < P;  // wave-uniform
   const int o0 = blockIdx.y * OW;
   const int li = lane & 15, lk = lane >> 4;
@@ -263,9 +269,10 @@ static bool two_tiles(int mt, long P, int n_orb) {
 template <typename TI, typename TO, int MT, int WPB, int PW>
 static void gemm_launch(const TI *Ct, int ldc, int n_orb, const TI *X, int ldk, long ldp, long P,
                         int kpad, const GemmOut &o, hipStream_t st) {
-  const unsigned gx = (unsigned)((P + 16 * PW * WPB - 1) / (16 * PW * WPB));
+  unsigned gx = (unsigned)((P + 16 * PW * WPB - 1) / (16 * PW * WPB));
+  if (o.out_val) gx = (gx + 7) / 8 * 8;  // whole turns of the XCDs
   hipLaunchKernelGGL((orbital_gemm_kernel<TI, TO, MT, WPB, PW>),
-                     dim3((gx + 7) / 8 * 8 * kComp, (unsigned)((n_orb + 16 * MT - 1) / (16 * MT))),
+                     dim3(gx * kComp, (unsigned)((n_orb + 16 * MT - 1) / (16 * MT))),
                      dim3(64 * WPB), 0, st, Ct, ldc, n_orb, X, ldk, ldp, P, kpad, o);
 }
 template <typename TI, typename TO, int WPB>
