@@ -11,11 +11,16 @@
 // QMCSCFJastrow::calculate_Psi_quantities / calculate_E_Local
 // (QMCSCFJastrow.cpp:196-282, QMCSCFJastrow.h:311-314).
 //
-// One workgroup per walker.  Every sum that reaches a gradient keeps the order
-// of a plain loop (orbitals ascending in a trace; nuclei, then partners
-// ascending in a Jastrow gradient), so that gradients, and the walks that
-// follow them, are bit for bit those of one thread an electron; sums that only
-// reach energies and ln Psi are added in any order.
+// One workgroup per walker, of four waves, up to 16 electrons of one: of a small
+// molecule four waves are mostly idle, and their LDS keeps all but three walkers
+// off a CU (all-electron moves, us a step with four and with one: 2 electrons x
+// 65536 walkers 1658 and 404, x 128 28.9 and 28.1; 10 x 16000 651 and 282).  For
+// 32 electrons one wave took a twentieth longer at 128 walkers.
+// Every sum that reaches a gradient keeps the order of a plain loop (orbitals
+// ascending in a trace; nuclei, then partners ascending in a Jastrow gradient), so
+// that gradients, and the walks that follow them, are bit for bit those of one
+// thread an electron; sums that only reach energies and ln Psi are added in any
+// order.
 #include "qmcb_ae.hpp"
 #include "qmcb_kernels.hpp"
 #include "qmcb_pade.hpp"
@@ -28,11 +33,13 @@ constexpr int kFN = 256;    // most electrons
 constexpr int kTile = 64;   // particles of a pair tile
 constexpr int kNuc = 40;    // nuclei of a tile (three workgroups' LDS on a CU)
 constexpr int kLd = kTile + 1;
+constexpr int kSmall = 16;  // most electrons (and nuclei of a tile) of the one-wave form
 
 template <typename TS>
 __device__ __forceinline__ double ldd(const TS *p) { return (double)*p; }
 
 struct JastrowLds {
+  static constexpr int kElectrons = kFN, kNuclei = kNuc;
   double x[kFN * 3];        // positions
   double g[3][kFN];         // Jastrow gradient
   double w[kTile * kLd];    // u'/r of a tile's pairs
@@ -40,6 +47,23 @@ struct JastrowLds {
   double en[2][kNuc][2];   // ... and of a tile's nuclei, by spin
   double nuc[kNuc * 3], z[kNuc];
 };
+
+// the one-wave form's: 6 KB
+struct SmallLds {
+  static constexpr int kElectrons = kSmall, kNuclei = kSmall;
+  double x[kSmall * 3], g[3][kSmall];
+  double w[kSmall * (kSmall + 1)];
+  double ee[3][2], en[2][kSmall][2];
+  double nuc[kSmall * 3], z[kSmall];
+};
+template <int FT>
+using FinishLds = std::conditional_t<FT == 64, SmallLds, JastrowLds>;
+
+// Squared distance, the products contracted as in a plain loop.
+__device__ __forceinline__ double dist2(const double *a, const double *b) {
+  const double dx = a[0] - b[0], dy = a[1] - b[1], dz = a[2] - b[2];
+  return __builtin_fma(dz, dz, __builtin_fma(dx, dx, dy * dy));
+}
 
 // Jastrow gradient of all electrons into L.g and, by thread, shares of U, its
 // Laplacian, V_ee and V_en (v[0..3]).  L.x holds the positions.  ONE: every Pade
@@ -72,10 +96,6 @@ __device__ __forceinline__ void jastrow_block(const DevSystem &S, JastrowLds &L,
     }
   };
   if (nn <= kNuc) load_en(0);
-  auto dist2 = [](const double *a, const double *b) {
-    const double dx = a[0] - b[0], dy = a[1] - b[1], dz = a[2] - b[2];
-    return __builtin_fma(dz, dz, __builtin_fma(dx, dx, dy * dy));
-  };
   // one coordinate of rows [r0, r0 + nr) gains `nc` partners at px, the pair's
   // value at w[row * sr + partner * sc]
   auto add = [&](int k, int r0, int nr, const double *px, int nc, int sr, int sc) {
@@ -151,23 +171,87 @@ __device__ __forceinline__ void jastrow_block(const DevSystem &S, JastrowLds &L,
   __syncthreads();
 }
 
+// The same for up to kSmall electrons by one wave: a lane a pair, then a lane a
+// coordinate of an electron, partners ascending.
+template <bool ONE>
+__device__ __forceinline__ void jastrow_block(const DevSystem &S, SmallLds &L, double v[4]) {
+  constexpr int LD = kSmall + 1;
+  const int t = threadIdx.x, N = S.N, nn = S.nn, nu = S.n[0];
+  const int k = t / kSmall, r = t % kSmall;  // coordinate k < 3 of electron r
+  auto add = [&](const double *px, int nc) {
+    if (k >= 3 || r >= N) return;
+    double g = L.g[k][r];
+    const double xr = L.x[3 * r + k];
+    for (int c = 0; c < nc; c++) g = __builtin_fma(L.w[r * LD + c], xr - px[3 * c + k], g);
+    L.g[k][r] = g;
+  };
+  if (k < 3) L.g[k][r] = 0.0;
+  if (ONE && t < 3) {
+    L.ee[t][0] = S.ee[t].num[0];
+    L.ee[t][1] = S.ee[t].den[0];
+  }
+  for (int a0 = 0; a0 < nn; a0 += kSmall) {
+    const int na = min(kSmall, nn - a0);
+    __syncthreads();
+    if (t < 3 * na) L.nuc[t] = S.nuc_xyz[3 * a0 + t];
+    if (t < na) L.z[t] = S.nuc_z[a0 + t];
+    if (ONE && k < 2 && r < na) {
+      L.en[k][r][0] = S.en[k][a0 + r].num[0];
+      L.en[k][r][1] = S.en[k][a0 + r].den[0];
+    }
+    __syncthreads();
+    for (int q = t; q < N * na; q += 64) {
+      const int i = q / na, a = q % na, sp = i < nu ? 0 : 1;
+      const double d = sqrt(dist2(L.x + 3 * i, L.nuc + 3 * a)), ir = 1.0 / d;
+      double u, du, d2u;
+      if constexpr (ONE) pade_first(L.en[sp][a], d, u, du, d2u);
+      else pade_eval(S.en[sp][a0 + a], d, u, du, d2u);
+      v[0] += u;
+      v[1] += 2.0 * ir * du + d2u;
+      v[3] -= L.z[a] * ir;
+      L.w[i * LD + a] = du * ir;
+    }
+    __syncthreads();
+    add(L.nuc, na);
+  }
+  __syncthreads();
+  if (t < N) L.w[t * LD + t] = 0.0;
+  // rows a and N - 1 - a together hold N - 1 pairs
+  for (int q = t; q < (N + 1) / 2 * (N - 1); q += 64) {
+    const int a = q / (N - 1), l = q % (N - 1), b = N - 1 - a;
+    if (l >= a && b == a) continue;
+    const int i = l < a ? a : b, j = l < a ? l : l - a;
+    const double d = sqrt(dist2(L.x + 3 * i, L.x + 3 * j)), ir = 1.0 / d;
+    double u, du, d2u;
+    if constexpr (ONE) pade_first(L.ee[ee_type(i, j, nu)], d, u, du, d2u);
+    else pade_eval(S.ee[ee_type(i, j, nu)], d, u, du, d2u);
+    v[0] += u;
+    v[1] += 2.0 * (2.0 * ir * du + d2u);
+    v[2] += ir;
+    L.w[i * LD + j] = L.w[j * LD + i] = du * ir;
+  }
+  __syncthreads();
+  add(L.x, N);
+  __syncthreads();
+}
+
 }  // namespace
 
 // all-electron Jastrow and potential alone (several determinants)
-template <bool ONE>
-__global__ void __launch_bounds__(kFT)
+template <bool ONE, int FT>
+__global__ void __launch_bounds__(FT)
 jastrow_all_kernel(JastrowArgs A, const int *walkers, int num) {
-  __shared__ JastrowLds L;
-  __shared__ double scratch[4][kFT / 64];
+  __shared__ FinishLds<FT> L;
+  __shared__ double scratch[4][FT / 64];
   const int b = blockIdx.x, t = threadIdx.x;
   if (b >= num) return;
   const int w = walkers ? walkers[b] : b, N = A.sys.N;
-  for (int i = t; i < 3 * N; i += kFT) L.x[i] = A.R[(long)w * N * 3 + i];
+  for (int i = t; i < 3 * N; i += FT) L.x[i] = A.R[(long)w * N * 3 + i];
   __syncthreads();
   double v[4] = {0.0, 0.0, 0.0, 0.0};
   jastrow_block<ONE>(A.sys, L, v);
   block_sums(v, scratch);
-  for (int i = t; i < 3 * N; i += kFT) A.Ux[(long)w * N * 3 + i] = L.g[i % 3][i / 3];
+  for (int i = t; i < 3 * N; i += FT) A.Ux[(long)w * N * 3 + i] = L.g[i % 3][i / 3];
   if (t == 0) {
     A.U[w] = v[0];
     A.Uxx[w] = v[1];
@@ -180,11 +264,13 @@ hipError_t launch_jastrow_all(const JastrowArgs &a, bool pade_one, const int *wa
                               hipStream_t st) {
   if (num <= 0) return hipSuccess;
   if (a.sys.N > kFN) return hipErrorInvalidValue;
-  if (pade_one)
-    hipLaunchKernelGGL((jastrow_all_kernel<true>), dim3(num), dim3(kFT), 0, st, a, walkers, num);
-  else
-    hipLaunchKernelGGL((jastrow_all_kernel<false>), dim3(num), dim3(kFT), 0, st, a, walkers, num);
-  return hipGetLastError();
+  auto launch = [&](auto kernel, int threads) {
+    hipLaunchKernelGGL(kernel, dim3(num), dim3(threads), 0, st, a, walkers, num);
+    return hipGetLastError();
+  };
+  if (a.sys.N <= kSmall)
+    return pade_one ? launch(jastrow_all_kernel<true, 64>, 64) : launch(jastrow_all_kernel<false, 64>, 64);
+  return pade_one ? launch(jastrow_all_kernel<true, kFT>, kFT) : launch(jastrow_all_kernel<false, kFT>, kFT);
 }
 
 // In place of two trace launches, Jastrow, assembly, decision and proposal: 700
@@ -193,15 +279,16 @@ hipError_t launch_jastrow_all(const JastrowArgs &a, bool pade_one, const int *wa
 // derivatives are 180 at the copy rate.
 //
 // What a small walker spends its time on here is loads in a row (2 electrons:
-// 41000 cycles when the decision read the outputs back), so everything that is
-// known at the start is loaded there: the record of the move, and by electron
-// (a thread each) the saved position and the drift it came from.
-template <typename TS, bool ONE>
-__global__ void __launch_bounds__(kFT) finish_kernel(FinishArgs F, const int *walkers, int num) {
-  static_assert(kFN <= kFT, "a thread an electron");
-  __shared__ JastrowLds L;
-  __shared__ double gs[kFN * 3];  // Slater gradient
-  __shared__ double scratch[8][kFT / 64];
+// waits are 78 % of the waves' cycles), so everything that is known at the start
+// is loaded there: the record of the move, and by electron (a thread each) the
+// saved position and the drift it came from.
+template <typename TS, bool ONE, int FT>
+__global__ void __launch_bounds__(FT) finish_kernel(FinishArgs F, const int *walkers, int num) {
+  typedef FinishLds<FT> Lds;
+  static_assert(Lds::kElectrons <= FT, "a thread an electron");
+  __shared__ Lds L;
+  __shared__ double gs[Lds::kElectrons * 3];  // Slater gradient
+  __shared__ double scratch[8][FT / 64];
   const int b = blockIdx.x, t = threadIdx.x;
   if (b >= num) return;
   const AssembleArgs &A = F.a;
@@ -209,7 +296,7 @@ __global__ void __launch_bounds__(kFT) finish_kernel(FinishArgs F, const int *wa
   const int w = walkers ? walkers[b] : b;
   const int N = S.N, nu = S.n[0];
   const double *Rw = A.R + (long)w * N * 3;
-  for (int i = t; i < 3 * N; i += kFT) L.x[i] = Rw[i];
+  for (int i = t; i < 3 * N; i += FT) L.x[i] = Rw[i];
   double logdet = 0.0, sgn = 1.0;
   bool sp_sing[2] = {false, false};
 #pragma unroll
@@ -235,7 +322,7 @@ __global__ void __launch_bounds__(kFT) finish_kernel(FinishArgs F, const int *wa
   // with four lanes an electron short rows keep the loads of 25-electron spins
   // in flight as well.  A singular walker keeps its resident gradient.
   double lap[2] = {0.0, 0.0};
-  for (int i = t; i < 4 * N; i += kFT) {
+  for (int i = t; i < 4 * N; i += FT) {
     const bool dn = i >= 4 * nu;
     const int n = dn ? S.n[1] : nu, e0 = dn ? nu : 0;
     const int q = i - 4 * e0, e = q >> 2, k = q & 3;
@@ -293,7 +380,7 @@ __global__ void __launch_bounds__(kFT) finish_kernel(FinishArgs F, const int *wa
       f = (-1.0 + sqrt(1.0 + 2 * A.umrigar_a * v[7] * A.dt)) / (A.umrigar_a * v[7] * A.dt);
     if (A.drift_mod == QMCB_DRIFT_UMRIGAR93_UNEQUAL) {
       const double x[3] = {L.x[3 * t], L.x[3 * t + 1], L.x[3 * t + 2]};
-      if (S.nn <= kNuc) f = drift_factor_unequal(g, x, S.nn, L.nuc, L.z, A.dt);
+      if (S.nn <= Lds::kNuclei) f = drift_factor_unequal(g, x, S.nn, L.nuc, L.z, A.dt);
       else f = drift_factor_unequal(g, x, S.nn, S.nuc_xyz, S.nuc_z, A.dt);
     }
     double *o = A.out.mod_drift + ((long)b * N + t) * 3;
@@ -357,11 +444,15 @@ hipError_t launch_finish(const FinishArgs &f, const int *walkers, int num, hipSt
   if (num <= 0) return hipSuccess;
   if (f.a.sys.N > kFN || f.a.s[0].ndet > 1 || f.a.s[0].occ || f.a.s[1].occ)
     return hipErrorInvalidValue;
-  if (f.pade_one)
-    hipLaunchKernelGGL((finish_kernel<TS, true>), dim3(num), dim3(kFT), 0, st, f, walkers, num);
-  else
-    hipLaunchKernelGGL((finish_kernel<TS, false>), dim3(num), dim3(kFT), 0, st, f, walkers, num);
-  return hipGetLastError();
+  auto launch = [&](auto kernel, int threads) {
+    hipLaunchKernelGGL(kernel, dim3(num), dim3(threads), 0, st, f, walkers, num);
+    return hipGetLastError();
+  };
+  if (f.a.sys.N <= kSmall)
+    return f.pade_one ? launch(finish_kernel<TS, true, 64>, 64)
+                      : launch(finish_kernel<TS, false, 64>, 64);
+  return f.pade_one ? launch(finish_kernel<TS, true, kFT>, kFT)
+                    : launch(finish_kernel<TS, false, kFT>, kFT);
 }
 template hipError_t launch_finish<double>(const FinishArgs &, const int *, int, hipStream_t);
 template hipError_t launch_finish<float>(const FinishArgs &, const int *, int, hipStream_t);

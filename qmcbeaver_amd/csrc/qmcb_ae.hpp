@@ -5,12 +5,17 @@
 
 namespace qmcb {
 
-constexpr int kAeT = 256;  // threads of a workgroup, a thread an electron
+constexpr int kAeT = 256;  // most threads of a workgroup, a thread an electron
 
-// v[k] summed over the workgroup (waves in order)
-template <int NV>
-__device__ __forceinline__ void block_sums(double (&v)[NV], double (*scratch)[kAeT / 64]) {
+// v[k] summed over the workgroup of NW waves (waves in order)
+template <int NV, int NW>
+__device__ __forceinline__ void block_sums(double (&v)[NV], double (*scratch)[NW]) {
   const int t = threadIdx.x;
+  if constexpr (NW == 1) {
+#pragma unroll
+    for (int k = 0; k < NV; k++) v[k] = wave_sum(v[k]);
+    return;
+  }
 #pragma unroll
   for (int k = 0; k < NV; k++) {
     const double s = wave_sum(v[k]);
@@ -20,7 +25,7 @@ __device__ __forceinline__ void block_sums(double (&v)[NV], double (*scratch)[kA
 #pragma unroll
   for (int k = 0; k < NV; k++) {
     double s = 0.0;
-    for (int q = 0; q < kAeT / 64; q++) s += scratch[k][q];
+    for (int q = 0; q < NW; q++) s += scratch[k][q];
     v[k] = s;
   }
   __syncthreads();
@@ -60,9 +65,10 @@ __device__ __forceinline__ double ae_propose_electron(const AeArgs &A, long step
 
 // The proposal of step `step` of walker w (batch row b) by a workgroup, a thread
 // an electron at x with drift f.
+template <int NW>
 __device__ __forceinline__ void ae_propose_block(const AeArgs &A, long step, int b, int w,
                                                  const double x[3], const double f[3],
-                                                 double (*scratch)[kAeT / 64]) {
+                                                 double (*scratch)[NW]) {
   const int t = threadIdx.x;
   double sq[1] = {0.0};
   if (t < A.N) sq[0] = ae_propose_electron(A, step, w, t, x, f);
