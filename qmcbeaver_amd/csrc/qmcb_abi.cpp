@@ -93,6 +93,7 @@ struct qmcb_ctx {
   int pade_mn = 0, pade_md = 0;   // most terms of any Pade function
   bool pade_one = true;           // every one has one term in each polynomial
   int np_shell = 0;               // primitives, each shell's counted once
+  const double *walk_tab = nullptr;  // the walk's tables (WalkArgs::tab)
   double *carry = nullptr;        // [Wc][walk_carry_len] block sums of the FP64 walk
   int *carried = nullptr;         // [Wc] (SlaterArgs)
   float *Cw[2] = {nullptr, nullptr};  // FP32 coefficients as [kpad / 4][npad][4]
@@ -840,6 +841,45 @@ WalkTables walk_tables(const qmcb_system *s, const Shells &sh) {
   return t;
 }
 
+// The walk's tables (WalkArgs::tab).
+std::vector<double> walk_table(const qmcb_system *s, const Shells &sh, const WalkTables &t) {
+  std::vector<double> out((size_t)walk_tab_len(s->n_basis, s->n_nuc, t.np, t.mn, t.md), 0.0);
+  double *prim = out.data(), *nuc = prim + 2 * t.np, *pade = nuc + 4 * s->n_nuc;
+  const int stride = 1 + t.mn + t.md;
+  auto put = [&](const qmcb_pade &f) {
+    const int64_t counts = ((int64_t)f.n_den << 32) | (int64_t)(uint32_t)f.n_num;
+    std::memcpy(pade, &counts, 8);
+    for (int i = 0; i < t.mn; i++) pade[1 + i] = f.num[i];
+    for (int i = 0; i < t.md; i++) pade[1 + t.mn + i] = f.den[i];
+    pade += stride;
+  };
+  for (const qmcb_pade *f : {&s->ee_updn, &s->ee_upup, &s->ee_dndn}) put(*f);
+  for (const qmcb_pade *en : {s->en_up, s->en_dn})
+    for (int i = 0; i < s->n_nuc; i++) put(en[i]);
+  for (int i = 0; i < s->n_nuc; i++) {
+    for (int k = 0; k < 3; k++) nuc[4 * i + k] = s->nuc_xyz[3 * i + k];
+    nuc[4 * i + 3] = s->nuc_z[i];
+  }
+  uint64_t *fn = (uint64_t *)pade;
+  int *atom = (int *)(fn + s->n_basis);
+  int p0 = 0;
+  for (size_t i = 0; i < sh.atom.size(); i++) {
+    const int np = sh.nprim[i];
+    for (int j = 0; j < np; j++) {
+      prim[2 * (p0 + j)] = s->prim_alpha[sh.prim_off[i] + j];
+      prim[2 * (p0 + j) + 1] = s->prim_coef[sh.prim_off[i] + j];
+      atom[p0 + j] = sh.atom[i];
+    }
+    for (int j = sh.bf0[i]; j < sh.bf0[i] + sh.ncart[i]; j++) {
+      const int *p = s->bf_pow + 3 * j;
+      fn[j] = (uint64_t)(p[0] | (p[1] << 2) | (p[2] << 4)) | (uint64_t)np << 6 |
+              (uint64_t)p0 << 22 | (uint64_t)sh.atom[i] << 44;
+    }
+    p0 += np;
+  }
+  return out;
+}
+
 // Whether a context's single-electron walk runs as walk_kernel (kpad, tx: padded
 // functions, bytes of the GEMM operand).  The environment's switches for kernels
 // of the step-by-step walk select that walk.
@@ -1039,6 +1079,10 @@ qmcb_status create_impl(const qmcb_system *s, const qmcb_options *o, qmcb_ctx *c
   }
 
   ctx->walk = walk_possible(s, o, sh, wt, ctx->kpad, ctx->tx);
+  if (ctx->walk) {
+    const std::vector<double> tab = walk_table(s, sh, wt);
+    QCHK(upload(ctx, &ctx->walk_tab, tab.data(), tab.size()));
+  }
 
   // ---- transposed, padded MO coefficients (active orbitals) in the operand type
   for (int sp = 0; sp < 2; sp++) {
@@ -1381,6 +1425,7 @@ size_t plan_device_bytes(const qmcb_system *s, const qmcb_options *o) {
   const long nkc = (B + kOrbChunk - 1) / kOrbChunk;
   const WalkTables wt = walk_tables(s, sh);
   const bool walks = walk_possible(s, o, sh, wt, (int)kpad, tx);
+  if (walks) add(walk_tab_len((int)B, (int)nn, wt.np, wt.mn, wt.md), 8);
   add(nshell, sizeof(OrbShell));
   add(nkc * kOrbChunk, sizeof(OrbFn));
   add(nkc, sizeof(int4));
@@ -1895,7 +1940,11 @@ static qmcb_status main_wait_groups(qmcb_ctx *ctx, int G) {
 // sweeps go to vrow, which no walk keeps anything in.
 static WalkArgs walk_args(qmcb_ctx *ctx, long first, int steps, double tau, int mode, int num) {
   WalkArgs a{};
-  a.sys = ctx->dsys;
+  a.nn = ctx->nn;
+  a.B = ctx->B;
+  a.nshell = ctx->nshell;
+  a.tab = ctx->walk_tab;
+  a.tab_len = walk_tab_len(ctx->B, ctx->nn, ctx->np_shell, ctx->pade_mn, ctx->pade_md);
   for (int sp = 0; sp < 2; sp++) {
     a.s[sp] = slater_args(ctx, sp);
     a.Ct[sp] = ctx->Ct[sp];

@@ -150,12 +150,13 @@ __device__ inline double reweight_walker(double wt, double dW, int age, double e
 // x: nearest nucleus, its charge and the time step (QMCSCFJastrow.cpp:368-443).
 // The nearest nucleus (first of equals) and the factor given it are split so
 // that callers evaluating two gradients at one position search once.
-__device__ inline int nearest_nucleus(const double x[3], int nn, const double *nuc_xyz) {
+__device__ inline int nearest_nucleus(const double x[3], int nn, const double *nuc_xyz,
+                                      int stride = 3) {
   int cn = 0;
   double best = 1e300;
   for (int A = 0; A < nn; A++) {
-    const double dx = x[0] - nuc_xyz[3 * A], dy = x[1] - nuc_xyz[3 * A + 1],
-                 dz = x[2] - nuc_xyz[3 * A + 2];
+    const double *p = nuc_xyz + stride * A;
+    const double dx = x[0] - p[0], dy = x[1] - p[1], dz = x[2] - p[2];
     const double r = sqrt(dx * dx + dy * dy + dz * dz);
     if (r < best) { best = r; cn = A; }
   }

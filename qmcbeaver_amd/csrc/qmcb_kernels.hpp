@@ -347,7 +347,6 @@ bool sm_move_fuses_jastrow(int n, int N);
 // determinant; walk.hip): step first_step + s moves electron (first_step + s)
 // mod N of every walker.
 struct WalkArgs {
-  DevSystem sys;
   SlaterArgs s[2];
   int N, n_up, nsteps;
   long first_step;
@@ -359,6 +358,12 @@ struct WalkArgs {
   int np;                // primitives, each shell's counted once
   int pade_mn, pade_md;  // most numerator / denominator terms of any Pade function
   int pade_one;          // every one has exactly one of each
+  // the system's tables in the order of the kernel's LDS (an even number of
+  // doubles): primitives {exponent, coefficient}, nuclei {x, y, z, Z}, Pade
+  // functions of electron pairs and of nuclei by spin, packed; a function's record;
+  // the atom of a primitive (ints)
+  int nn, B, nshell, tab_len;
+  const double *tab;
   int has_cusp;
   CuspDev cusp[2];
   double *R, *U, *Ux, *Uxx, *Vee, *Ven, *cur_el;
@@ -379,6 +384,11 @@ struct WalkArgs {
   double *carry;
   int keep;
 };
+// doubles of WalkArgs::tab, even
+inline int walk_tab_len(int B, int nn, int np, int mn, int md) {
+  const int n = 2 * np + 4 * nn + (3 + 2 * nn) * (1 + mn + md) + B + (np + 1) / 2;
+  return (n + 1) / 2 * 2;
+}
 // doubles of WalkArgs::carry a walker (0: none are kept)
 long walk_carry_len(int n_up, size_t tx);
 template <typename TS, typename TX>

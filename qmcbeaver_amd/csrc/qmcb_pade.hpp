@@ -51,10 +51,5 @@ __device__ __forceinline__ void pade_first(const double *f, double r, double &u,
   du = __builtin_fma(-u, bp, ap) * ib;
   d2u = -(2.0 * du * bp) * ib;
 }
-__device__ __forceinline__ void pade_pack(double *dst, const PadeShape &ps, const qmcb_pade &f) {
-  dst[0] = __builtin_bit_cast(double, ((long long)f.n_den << 32) | (long long)(unsigned)f.n_num);
-  for (int i = 0; i < ps.mn; i++) dst[1 + i] = f.num[i];
-  for (int i = 0; i < ps.md; i++) dst[1 + ps.mn + i] = f.den[i];
-}
 
 }  // namespace qmcb

@@ -240,8 +240,7 @@ walk_kernel(WalkArgs A, const int *walkers, int num) {
   const int w = walkers ? walkers[b] : b;
   const int t = threadIdx.x, lane = t & 63, wave = __builtin_amdgcn_readfirstlane(t >> 6);
   const int grp = NG > 1 ? wave / (NW / NG) : 0, c = t % (NC * SL) / SL, sl = t % SL;
-  const DevSystem &S = A.sys;
-  const int N = A.N, nu = A.n_up, nn = S.nn, B = S.B, nshell = S.nshell, kpad = A.kpad;  // FP32: a multiple of 48
+  const int N = A.N, nu = A.n_up, nn = A.nn, B = A.B, kpad = A.kpad;  // FP32: a multiple of 48
   const PadeShape ps{A.pade_mn, A.pade_md};
   const int PS = ps.stride();
   const double tau = A.tau;
@@ -260,56 +259,28 @@ walk_kernel(WalkArgs A, const int *walkers, int num) {
   __shared__ double s_psi[2][3];  // U and ln|det| of either spin, by step parity
   extern __shared__ __align__(16) unsigned char dyn[];
   TX *X = (TX *)dyn;                                     // basis values, x_words(kpad) values
+  // tables, in the order of WalkArgs::tab
   double *s_prim = (double *)(X + (size_t)kpad * kXWords<TX>);  // [np]{exponent, coefficient}
-  double *s_ex = s_prim + 2 * A.np;                      // [np] exponentials
-  double *s_nuc = s_ex + A.np;                           // [nn]{x, y, z, Z}
-  double *s_rn = s_nuc + 4 * nn;                         // distance of the proposal to each nucleus
-  double *s_ee = s_rn + nn;                              // [3][PS]
+  double *s_nuc = s_prim + 2 * A.np;                     // [nn]{x, y, z, Z}
+  double *s_ee = s_nuc + 4 * nn;                         // [3][PS]
   double *s_en = s_ee + 3 * PS;                          // [2][nn][PS]
-  double *s_blk = s_en + 2 * nn * PS;                    // not RD: [NC][KB] columns of A^-1
-  double *s_vrow = s_blk + (RD ? 0 : NC * KB);           // not RD: [KB][NC][4] rows replaced
-  uint64_t *s_fn = (uint64_t *)(s_vrow + (RD ? 0 : KB * NC * 4));  // [B] function records
+  uint64_t *s_fn = (uint64_t *)(s_en + 2 * nn * PS);     // [B] function records
   int *s_pa = (int *)(s_fn + B);                         // [np] atom of a primitive
-  int *s_off = s_pa + A.np;                              // [nshell + 1] shells' first primitives
+  // scratch
+  double *s_ex = (double *)(s_fn + B) + (A.np + 1) / 2;  // [np] exponentials
+  double *s_rn = s_ex + A.np;                            // distance of the proposal to each nucleus
+  double *s_blk = s_rn + nn;                             // not RD: [NC][KB] columns of A^-1
+  double *s_vrow = s_blk + (RD ? 0 : NC * KB);           // not RD: [KB][NC][4] rows replaced
 
-  // ---- tables: nuclei, Pade functions, primitives once per shell, functions
-  for (int i = t; i < nn; i += NT) {
-    for (int k = 0; k < 3; k++) s_nuc[4 * i + k] = S.nuc_xyz[3 * i + k];
-    s_nuc[4 * i + 3] = S.nuc_z[i];
-    for (int s = 0; s < 2; s++) pade_pack(s_en + (s * nn + i) * PS, ps, S.en[s][i]);
+  // the tables as the host laid them out (formed here from the system's arrays, a
+  // chain of dependent loads, they were half of a launch of one step)
+  {
+    typedef double d2v __attribute__((ext_vector_type(2)));
+    for (int i = t; 2 * i < A.tab_len; i += NT) ((d2v *)s_prim)[i] = ((const d2v *)A.tab)[i];
   }
-  if (t < 3) pade_pack(s_ee + t * PS, ps, S.ee[t]);
   for (int i = t; i < kpad * kXWords<TX>; i += NT) X[i] = (TX)0;
   for (int i = t; i < kComp * NC; i += NT) s_v[0][i] = 0.0;
   for (int i = t; i < 2 * NC; i += NT) s_col[0][i] = 0.0;
-  if (wave == 0) {  // first primitive of each shell: a scan by the first wave
-    int base = 0;
-    for (int i0 = 0; i0 < nshell; i0 += 64) {
-      int v = i0 + lane < nshell ? S.sh_nprim[i0 + lane] : 0;
-      for (int d = 1; d < 64; d <<= 1) {
-        const int u = __shfl_up(v, d, 64);
-        if (lane >= d) v += u;
-      }
-      if (i0 + lane < nshell) s_off[i0 + lane + 1] = base + v;
-      base += __shfl(v, 63, 64);
-    }
-    if (lane == 0) s_off[0] = 0;
-  }
-  __syncthreads();
-  for (int i = t; i < nshell; i += NT) {
-    const int nc = S.sh_ncart[i], bf0 = S.sh_bf0[i], np = S.sh_nprim[i], p0 = s_off[i];
-    const int at = S.sh_atom[i], g0 = S.sh_prim_off[i];
-    for (int j = 0; j < np; j++) {
-      s_prim[2 * (p0 + j)] = S.prim_alpha[g0 + j];
-      s_prim[2 * (p0 + j) + 1] = S.prim_coef[g0 + j];
-      s_pa[p0 + j] = at;
-    }
-    for (int j = 0; j < nc; j++) {
-      const int *p = S.bf_pow + 3 * (bf0 + j);
-      s_fn[bf0 + j] = (uint64_t)(p[0] | (p[1] << 2) | (p[2] << 4)) | (uint64_t)np << 6 |
-                      (uint64_t)p0 << 22 | (uint64_t)at << 44;
-    }
-  }
 
   // ---- walker state: thread e < N holds electron e's position, Jastrow and
   // determinant gradients, drift factor and nearest nucleus
@@ -347,10 +318,11 @@ walk_kernel(WalkArgs A, const int *walkers, int num) {
     s_sc[15] = A.acc_prop_el[w];
     if (A.mode == 2) s_sc[16] = A.acc_w[w];
   }
+  __syncthreads();
   if (qf && t < N) {
     double v[3];
     for (int k = 0; k < 3; k++) v[k] = ge[k] + Ue[k];
-    cn = nearest_nucleus(Re, nn, S.nuc_xyz);
+    cn = nearest_nucleus(Re, nn, s_nuc, 4);
     fo = drift_factor_lds(v, Re, s_nuc + 4 * cn, tau);
   }
 
@@ -1220,7 +1192,8 @@ walk_kernel(WalkArgs A, const int *walkers, int num) {
 
 namespace {
 
-// dynamic LDS of the launch: basis values and tables (walk_kernel's layout)
+// dynamic LDS of the launch: basis values, tables and scratch (walk_kernel's
+// layout; the last term of the sum is more than its rounding to even lengths)
 size_t walk_lds(int NC, int B, int kpad, int nn, int nshell, int np, int mn, int md, size_t tx) {
   const size_t ps = 1 + mn + md;
   size_t d = 3 * (size_t)np + 5 * (size_t)nn + (3 + 2 * (size_t)nn) * ps + (size_t)B;
@@ -1260,8 +1233,8 @@ long walk_carry_len(int n_up, size_t tx) {
 
 template <typename TS, typename TX, int NC>
 static hipError_t launch_tile(const WalkArgs &a, const int *walkers, int num, hipStream_t st) {
-  const size_t lds = walk_lds(NC, a.sys.B, a.kpad, a.sys.nn, a.sys.nshell, a.np, a.pade_mn,
-                              a.pade_md, sizeof(TX));
+  const size_t lds = walk_lds(NC, a.B, a.kpad, a.nn, a.nshell, a.np, a.pade_mn, a.pade_md,
+                              sizeof(TX));
   auto k = walk_kernel<TS, TX, NC>;
   if (lds > 48 * 1024) {
     const hipError_t e = hipFuncSetAttribute((const void *)k, hipFuncAttributeMaxDynamicSharedMemorySize,
@@ -1275,8 +1248,10 @@ static hipError_t launch_tile(const WalkArgs &a, const int *walkers, int num, hi
 template <typename TS, typename TX>
 hipError_t launch_walk(const WalkArgs &a, const int *walkers, int num, hipStream_t st) {
   if (num <= 0 || a.nsteps <= 0) return hipSuccess;
-  if (!walk_fits(a.n_up, a.N - a.n_up, a.sys.B, a.kpad, a.sys.nn, a.sys.nshell, a.np, a.pade_mn, a.pade_md,
+  if (!walk_fits(a.n_up, a.N - a.n_up, a.B, a.kpad, a.nn, a.nshell, a.np, a.pade_mn, a.pade_md,
                  sizeof(TX)) ||
+      !a.tab || a.tab_len % 2 != 0 ||
+      a.tab_len < walk_tab_len(a.B, a.nn, a.np, a.pade_mn, a.pade_md) ||
       a.N > 2 * a.n_up || (walk_carry_len(a.n_up, sizeof(TX)) > 0 && (!a.carry || !a.s[0].carried)))
     return hipErrorInvalidValue;
   const int NC = walk_tile(a.n_up);
