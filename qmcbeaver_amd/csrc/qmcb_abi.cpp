@@ -2021,10 +2021,38 @@ static int walk_run_length(const qmcb_ctx *ctx, long first, long left, int num) 
 // walkers, 312 against 237 at 4000).  There both ways form a walker's
 // proposals, matrices and gradients with the same bits; the energies and
 // probabilities, whose sums are in another order, agree to rounding.  With FP64
-// operands everything does, and the choice is the system's alone.
+// operands everything does, and beyond 32 electrons a spin the choice is the
+// system's alone.
 constexpr int kWalkRounds64 = 4 * 256;
+// phase length S of the staggered re-inversion (refresh_plan)
+constexpr int kRefreshBatch = 1024;
+static int refresh_phase(int K, int num) {
+  return std::max(1, std::min(K, (int)(((long)K * kRefreshBatch + std::max(num, 1) - 1) /
+                                       std::max(num, 1))));
+}
+// Up to 32 electrons a spin, large batches whose phases of the staggered
+// re-inversion are short: a run of S steps reads and writes a walker's whole
+// state, which costs such a batch as much as S to 2 S steps, while the launches it
+// saves are hidden.  us a step, steps against runs: 8192 walkers of 38 electrons
+// FP32, S = 1 (K 4) 176 / 229, S = 2 136 / 163, S = 4 123 / 135, S = 8 116 / 120,
+// and of 4096 S = 1 121 / 137, S = 2 95 / 94; FP64 (its steps take twice the
+// time) 8192 S = 1 179 / 203, S = 2 153 / 148, 4096 S = 1 130 / 125; 2 electrons,
+// S = 1, 65536 walkers 481 / 538 FP32 and 489 / 524 FP64, 32768 261 / 281 and
+// 264 / 272, 16384 150 / 150 and 150 / 145.  Where every step (FP64: every second)
+// re-inverts all walkers, the runs are level or ahead.  The choice rests on what
+// the schedule of re-inversions rests on, K and the batch, never on where calls,
+// windows or groups cut the walk.
+static bool short_phases(const qmcb_ctx *ctx, int num) {
+  const int K = ctx->opt.refresh_interval, n = ctx->n[0];
+  if (K < 2 || n > 32) return false;
+  const int S = refresh_phase(K, num);
+  if (n <= 16) return S == 1 && num >= 32768;
+  if (ctx->tx == 8) return S == 1 && K > 2 && num >= 6144;
+  return num >= 2048 * std::max(S, 2);
+}
 static bool walk_runs(const qmcb_ctx *ctx, int num) {
-  return ctx->walk && (ctx->tx == 8 || ctx->n[0] <= 32 || num <= kWalkRounds64);
+  return ctx->walk && (ctx->tx == 8 || ctx->n[0] <= 32 || num <= kWalkRounds64) &&
+         !short_phases(ctx, num);
 }
 
 // the counts of moves_of_spin after a run: every step but its last (which the
@@ -2072,11 +2100,6 @@ static qmcb_status series_reserve(qmcb_ctx *ctx, int64_t first_step, int32_t n_s
 // share of a walker group (a contiguous range of list positions) is a
 // contiguous piece of rmap.  rmap is copied to d_rmap; the caller
 // synchronises the stream before rmap changes again.
-constexpr int kRefreshBatch = 1024;
-static int refresh_phase(int K, int num) {
-  return std::max(1, std::min(K, (int)(((long)K * kRefreshBatch + std::max(num, 1) - 1) /
-                                       std::max(num, 1))));
-}
 static qmcb_status refresh_plan(qmcb_ctx *ctx, const int *slots, int num) {
   const int K = ctx->opt.refresh_interval;
   const int S = refresh_phase(K, num);
