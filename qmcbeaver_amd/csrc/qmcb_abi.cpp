@@ -2021,8 +2021,8 @@ static int walk_run_length(const qmcb_ctx *ctx, long first, long left, int num) 
 // walkers, 312 against 237 at 4000).  There both ways form a walker's
 // proposals, matrices and gradients with the same bits; the energies and
 // probabilities, whose sums are in another order, agree to rounding.  With FP64
-// operands everything does, and beyond 32 electrons a spin the choice is the
-// system's alone.
+// operands everything does, and no rule takes it from one way to the other but
+// the schedule of re-inversions (short_phases).
 constexpr int kWalkRounds64 = 4 * 256;
 // phase length S of the staggered re-inversion (refresh_plan)
 constexpr int kRefreshBatch = 1024;
@@ -2030,23 +2030,28 @@ static int refresh_phase(int K, int num) {
   return std::max(1, std::min(K, (int)(((long)K * kRefreshBatch + std::max(num, 1) - 1) /
                                        std::max(num, 1))));
 }
-// Up to 32 electrons a spin, large batches whose phases of the staggered
-// re-inversion are short: a run of S steps reads and writes a walker's whole
-// state, which costs such a batch as much as S to 2 S steps, while the launches it
-// saves are hidden.  us a step, steps against runs: 8192 walkers of 38 electrons
-// FP32, S = 1 (K 4) 176 / 229, S = 2 136 / 163, S = 4 123 / 135, S = 8 116 / 120,
-// and of 4096 S = 1 121 / 137, S = 2 95 / 94; FP64 (its steps take twice the
-// time) 8192 S = 1 179 / 203, S = 2 153 / 148, 4096 S = 1 130 / 125; 2 electrons,
-// S = 1, 65536 walkers 481 / 538 FP32 and 489 / 524 FP64, 32768 261 / 281 and
-// 264 / 272, 16384 150 / 150 and 150 / 145.  Where every step (FP64: every second)
-// re-inverts all walkers, the runs are level or ahead.  The choice rests on what
-// the schedule of re-inversions rests on, K and the batch, never on where calls,
+// Large batches whose phases of the staggered re-inversion are short walk step by
+// step: a run of S steps reads and writes a walker's whole state, which costs such a
+// batch as much as S to 2 S steps, while the launches it saves are hidden.  us a
+// step, steps against runs: 8192 walkers of 38 electrons FP32, S = 1 (K 4)
+// 176 / 229, S = 2 136 / 163, S = 4 123 / 135, S = 8 116 / 120, and of 4096 S = 1
+// 121 / 137, S = 2 95 / 94; FP64 (its steps take twice the time) 8192 S = 1
+// 179 / 203, S = 2 153 / 148, 4096 S = 1 130 / 125; 2 electrons, S = 1, 65536
+// walkers 481 / 538 FP32 and 489 / 524 FP64, 32768 261 / 281 and 264 / 272, 16384
+// 150 / 150 and 150 / 145.  Up to 32 electrons a spin and K 1 (FP64: 2) the runs
+// are level or ahead.  FP64 operands beyond 32, S = 1: 66 electrons x 1000 walkers
+// 197 / 176, x 4000 512 / 587, 100 x 1000 262 / 228, x 2000 401 / 420, 150 x 1000
+// 400 / 423, 256 x 500 470 / 445, x 1000 771 / 842; S = 2: 66 x 4000 241 / 269,
+// 100 x 4000 349 / 353, 256 x 2000 949 / 915.  The choice rests on what the
+// schedule of re-inversions rests on, K and the batch, never on where calls,
 // windows or groups cut the walk.
 static bool short_phases(const qmcb_ctx *ctx, int num) {
   const int K = ctx->opt.refresh_interval, n = ctx->n[0];
-  if (K < 2 || n > 32) return false;
+  if (K < 1 || (K == 1 && n <= 32)) return false;
   const int S = refresh_phase(K, num);
   if (n <= 16) return S == 1 && num >= 32768;
+  if (n > 32)
+    return ctx->tx == 8 && S <= (n <= 64 ? 2 : 1) && (long)num * n >= 65000L * S;
   if (ctx->tx == 8) return S == 1 && K > 2 && num >= 6144;
   return num >= 2048 * std::max(S, 2);
 }

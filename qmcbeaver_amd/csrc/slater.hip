@@ -1188,6 +1188,7 @@ sm_move_kernel(MoveArgs A, const int *walkers, int num) {
     A.s.dcount[w] = 0;
   }
   if (t == 0) {
+    if (sizeof(TO) == 8 && A.s.carried) A.s.carried[w] = 0;
     const double el = accept ? EL : el_old;
     if (A.walk.age) A.walk.age[w] = age_new;
     double wt = 1.0;
