@@ -8,8 +8,8 @@
 // orbital_gemm_kernel, the same bits: FP64 functions by shells, rounded to the
 // operand type, contracted in ascending function order by 16x16x4 MFMA.
 //
-// For batches too small to fill the chip twice over, where the two kernels are
-// chains of dependent loads on a few waves a SIMD: a workgroup holds a tile of
+// For batches of at most a workgroup a CU, where the two kernels are chains of
+// dependent loads on a few waves a SIMD: a workgroup holds a tile of
 // 16 points and up to 4 orbital tiles of 16, and runs four stages on successive
 // chunks of 32 functions, one barrier a chunk.  Waves 0-7 form the exponentials
 // of one chunk's primitives (a lane: one primitive at one point) and the radial
@@ -22,11 +22,12 @@
 // 128 walkers of 2 electrons 15 -> 7.5 us.
 //
 // Measured, FP32 operands: 1500 points x 75 orbitals x 804 functions 45 us
-// (basis 27 + contraction 39 before), 512 x 100 x 1019 59 us (35 + 52).  A
-// chunk takes about 4000 cycles, near the instruction issue of its stages (on
-// this card MFMA and FP64 vector work of one SIMD add rather than overlap:
-// roughly 730 exponentials, 1200 functions, 1300 MFMA), which is also why the
-// kernel gains nothing once the batch fills the chip.
+// (basis 27 + contraction 39 before), 512 x 100 x 1019 59 us (35 + 52).  In the
+// latter a chunk takes 3900 cycles, of which the matrix cores are busy 1050 and a
+// SIMD issues about 490 vector instructions, FP64 most of them and four cycles
+// each: the two add up on this card rather than overlap, which is also why the
+// kernel gains nothing once the batch fills the chip.  With FP64 operands 7
+// registers are spilled.
 #include <hip/hip_bf16.h>
 
 #include <algorithm>
