@@ -213,8 +213,9 @@ int32_t qmcb_abi_version(void);
  * step, 0 draws the next proposal inside the move kernel (same bits).  With
  * either variable set the device walk runs step by step; without, one kernel
  * carries the walkers of most systems of one determinant through a run of
- * steps: with FP32 operands the same positions bit for bit (17 to 32 up and 1
- * to 16 down electrons: to rounding), with FP64 ones to rounding. */
+ * steps, but for large batches that re-invert every few moves: with FP32
+ * operands the same positions bit for bit (17 to 32 up and 1 to 16 down
+ * electrons: to rounding), with FP64 ones to rounding. */
 qmcb_status qmcb_create(const qmcb_system *sys, const qmcb_options *opt,
                         qmcb_ctx **out);
 
